@@ -40,6 +40,7 @@ extern "C" {
 #define OW_FUSE_NORM 1     /* x is raw; apply the block's RMSNorm (omniweave/models/block.py:83-85) */
 #define OW_FUSE_RESIDUAL 2 /* write x + delta instead of delta (omniweave/models/block.py:108) */
 #define OW_FUSE_FP8 4      /* fp8-e4m3 channel side with ow_pack_weights_fp8 weights (needs OW_FUSE_NORM) */
+#define OW_WEIGHTS_X3 8    /* fp32 activations with ow_pack_weights_x3 weights (bf16 matrix cores, three-part operands) */
 
 /*
  * Route plan descriptor: the arguments of build_route_plan
@@ -115,6 +116,23 @@ int ow_pack_weights(const void* a_u, const void* a_v, const void* a_o,
                     const int32_t* channel_index, int32_t channels,
                     int32_t g, int32_t q_c, int32_t d, int32_t rd,
                     int32_t compute_dtype, void* packed, void* stream);
+
+/*
+ * Weights for fp32 activations on the bf16 matrix cores (flag OW_WEIGHTS_X3): every folded
+ * weight as three bf16 parts that sum to its 24 significand bits, in MFMA operand order.  The
+ * arguments and folds are ow_pack_weights' (compute dtype fp32); `packed` holds
+ * ow_packed_weight_bytes_x3(q_c, d, rd) bytes (6 per weight) and is 16-byte aligned.
+ * ow_weights_x3_supported: 1 when a plan's images lie within that kernel's 32-bit offsets (two
+ * images, or as many as 8 token groups span, below 1 GiB of fp32), else 0; larger images take
+ * ow_pack_weights' fp32 layout.
+ */
+int32_t ow_weights_x3_supported(const OwPlan* plan);
+size_t ow_packed_weight_bytes_x3(int32_t q_c, int32_t d, int32_t rd);
+int ow_pack_weights_x3(const void* a_u, const void* a_v, const void* a_o,
+                       const void* b_u, const void* b_v, const void* b_o,
+                       int32_t weight_dtype, const float* norm_weight, const float* gamma,
+                       const int32_t* channel_index, int32_t channels,
+                       int32_t g, int32_t q_c, int32_t d, int32_t rd, void* packed, void* stream);
 
 /*
  * fp8 inference variant (no counterpart in the reference, which has no fp8 path): the

@@ -12,6 +12,7 @@ OW_OK = 0
 OW_ROUTE = {"local": 0, "shifted": 1, "radix": 2}
 OW_DTYPE_F32, OW_DTYPE_BF16, OW_DTYPE_F16 = 0, 1, 2
 OW_FUSE_NORM, OW_FUSE_RESIDUAL, OW_FUSE_FP8 = 1, 2, 4
+OW_WEIGHTS_X3 = 8
 
 _c_int32_p = ctypes.POINTER(ctypes.c_int32)
 
@@ -40,6 +41,13 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_void_p] * 6 + [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]
         + [ctypes.c_int32] * 5 + [ctypes.c_void_p, ctypes.c_void_p],
+    ),
+    "ow_weights_x3_supported": (ctypes.c_int32, [ctypes.POINTER(OwPlan)]),
+    "ow_packed_weight_bytes_x3": (ctypes.c_size_t, [ctypes.c_int32] * 3),
+    "ow_pack_weights_x3": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 6 + [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]
+        + [ctypes.c_int32] * 4 + [ctypes.c_void_p, ctypes.c_void_p],
     ),
     "ow_packed_weight_bytes_fp8": (ctypes.c_size_t, [ctypes.c_int32] * 3),
     "ow_pack_weights_fp8": (

@@ -1269,6 +1269,36 @@ int ow_pack_weights(const void* a_u, const void* a_v, const void* a_o, const voi
   return OW_OK;
 }
 
+int32_t ow_weights_x3_supported(const OwPlan* plan) {
+  int32_t q_s = 0, q_c = 0;
+  if (ow_plan_dims(plan, &q_s, &q_c) != OW_OK) return 0;
+  return ow::x3_fits(plan->height * plan->width, plan->channels, q_s) ? 1 : 0;
+}
+
+size_t ow_packed_weight_bytes_x3(int32_t q_c, int32_t d, int32_t rd) {
+  if (q_c < 1 || (d != 64 && d != 128) || (rd != 128 && rd != 256)) return 0;
+  return ow::packed_bytes_x3(q_c, d, rd);
+}
+
+int ow_pack_weights_x3(const void* a_u, const void* a_v, const void* a_o, const void* b_u, const void* b_v,
+                       const void* b_o, int32_t weight_dtype, const float* norm_weight, const float* gamma,
+                       const int32_t* channel_index, int32_t channels, int32_t g, int32_t q_c, int32_t d, int32_t rd,
+                       void* packed, void* stream) {
+  OW_CHECK_ARG(a_u && a_v && a_o && b_u && b_v && b_o && packed, "weight or output pointer is NULL");
+  OW_CHECK_ARG(!(norm_weight || gamma) || channel_index, "norm_weight / gamma need channel_index");
+  OW_CHECK_ARG(weight_dtype >= OW_DTYPE_F32 && weight_dtype <= OW_DTYPE_F16, "unknown weight dtype %d", weight_dtype);
+  OW_CHECK_SUPPORTED(g == ow::kG, "unsupported spatial tile g=%d; expected 16", g);
+  OW_CHECK_ARG(q_c >= 1 && channels >= 1, "bad shape q_c=%d channels=%d", q_c, channels);
+  OW_CHECK_SUPPORTED((d == 64 || d == 128) && (rd == 128 || rd == 256),
+                     "unsupported channel tile d=%d / expanded dim rd=%d", d, rd);
+  OW_CHECK_ARG(ow::aligned16(packed), "packed weights must be 16-byte aligned");
+  if (int rc = ow::pack_weights_x3(a_u, a_v, a_o, b_u, b_v, b_o, weight_dtype, norm_weight, gamma, channel_index,
+                                   channels, q_c, d, rd, packed, static_cast<hipStream_t>(stream)))
+    return rc;
+  ow::clear_error();
+  return OW_OK;
+}
+
 size_t ow_packed_weight_bytes_fp8(int32_t q_c, int32_t d, int32_t rd) {
   if (q_c < 1 || d < 32 || rd < 32 || d % 32 || rd % 32) return 0;
   return static_cast<size_t>(ow::kF8HeadBytes) +
@@ -1359,16 +1389,20 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
   if (int rc = ow_plan_dims(plan, &q_s, &q_c)) return rc;
   OW_CHECK_ARG(batch >= 0, "batch must be >= 0 (got %d)", batch);
   OW_CHECK_ARG(packed && token_index && channel_index, "tensor pointer is NULL");
-  OW_CHECK_ARG((flags & ~(OW_FUSE_NORM | OW_FUSE_RESIDUAL | OW_FUSE_FP8)) == 0, "unknown flags 0x%x", flags);
+  OW_CHECK_ARG((flags & ~(OW_FUSE_NORM | OW_FUSE_RESIDUAL | OW_FUSE_FP8 | OW_WEIGHTS_X3)) == 0, "unknown flags 0x%x", flags);
   const bool fp8 = (flags & OW_FUSE_FP8) != 0;
   const bool norm = (flags & OW_FUSE_NORM) != 0;
+  const bool x3 = (flags & OW_WEIGHTS_X3) != 0;
+  OW_CHECK_SUPPORTED(!x3 || dtype == OW_DTYPE_F32, "OW_WEIGHTS_X3 needs f32 activations");
   OW_CHECK_SUPPORTED(!fp8 || (norm && dtype != OW_DTYPE_F32),
                      "OW_FUSE_FP8 needs OW_FUSE_NORM and bf16 / f16 activations");
   OW_CHECK_SUPPORTED(plan->spatial_tile == ow::kG, "unsupported spatial tile g=%d; expected 16", plan->spatial_tile);
   OW_CHECK_SUPPORTED(dtype == OW_DTYPE_BF16 || dtype == OW_DTYPE_F16 || dtype == OW_DTYPE_F32,
                      "unsupported dtype %d; expected bf16, f16 or f32", dtype);
   const int32_t n = plan->height * plan->width, c = plan->channels, d = plan->channel_tile;
-  const size_t want = fp8 ? ow_packed_weight_bytes_fp8(q_c, d, rd) : ow_packed_weight_bytes(q_c, d, rd, dtype);
+  const size_t want = fp8  ? ow_packed_weight_bytes_fp8(q_c, d, rd)
+                      : x3 ? ow_packed_weight_bytes_x3(q_c, d, rd)
+                           : ow_packed_weight_bytes(q_c, d, rd, dtype);
   OW_CHECK_ARG(want != 0 && packed_bytes == want,
                "packed weights hold %zu bytes; q_c=%d d=%d rd=%d needs %zu", packed_bytes, q_c, d, rd, want);
   OW_CHECK_ARG(ow::aligned16(packed), "packed weights must be 16-byte aligned");
@@ -1405,6 +1439,14 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
     if (want_scales) *scale_written = 1;
   }
 
+  if (x3) {
+    if (int rc = ow::launch_fwd_x3(static_cast<const float*>(x), static_cast<float*>(out), scale, packed, token_index,
+                                   channel_index, batch, n, c, q_s, q_c, d, rd, (flags & OW_FUSE_RESIDUAL) ? 1 : 0,
+                                   drop_scale, s))
+      return rc;
+    ow::clear_error();
+    return OW_OK;
+  }
   if (fp32) {
     if (int rc = ow::launch_fwd_f32(static_cast<const float*>(x), static_cast<float*>(out), scale,
                                     static_cast<const float*>(packed), token_index, channel_index, batch, n, c, q_s,

@@ -2,7 +2,9 @@
 // reference backend's fp32 semantics, omniweave/ops/reference.py:120-173, with the block's
 // RMSNorm prologue and residual epilogue of omniweave/models/block.py:83-108).
 //
-// One workgroup per tile (image b, token group s, channel group q), 256 threads, fp32 FMAs
+// Activations whose images lie beyond the matrix-core kernel's 32-bit offsets (bigemm_fwd_x3.hip
+// serves the rest, 3 to 5 times as fast), and callers of the C ABI with ow_pack_weights' fp32
+// layout.  One workgroup per tile (image b, token group s, channel group q), 256 threads, fp32 FMAs
 // staged through LDS:
 //   T = routed [16, d] tile of x (x * r with the RMSNorm, pads 0)
 //   P_u = A_u T, P_v = A_v T                     [16, d]

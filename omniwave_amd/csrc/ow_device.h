@@ -239,6 +239,10 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Waits for this wave's outstanding LDS reads, also those issued as inline assembly (before a
+// barrier that lets other waves overwrite what they read).
+__device__ __forceinline__ void wait_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // LDS byte address of a pointer into __shared__ memory.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
@@ -836,6 +840,17 @@ int rms_scale_f32(const float* x, float* scale, int64_t rows, int32_t channels, 
 int launch_fwd_f32(const float* x, float* out, const float* row_scale, const float* packed, const int32_t* tok,
                    const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s, int32_t q_c,
                    int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream);
+
+// fp32 path on the bf16 matrix cores (bigemm_fwd_x3.hip): three-part operands (ow_x3.h).
+bool x3_fits(int32_t n_tok, int32_t channels, int32_t q_s);  // images within its 32-bit offsets
+size_t packed_bytes_x3(int32_t q_c, int32_t d, int32_t rd);
+int pack_weights_x3(const void* a_u, const void* a_v, const void* a_o, const void* b_u, const void* b_v,
+                    const void* b_o, int32_t weight_dtype, const float* norm_weight, const float* gamma,
+                    const int32_t* channel_index, int32_t channels, int32_t q_c, int32_t d, int32_t rd, void* packed,
+                    hipStream_t stream);
+int launch_fwd_x3(const float* x, float* out, const float* row_scale, const void* packed, const int32_t* tok,
+                  const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s, int32_t q_c,
+                  int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream);
 
 // fp32 backward building blocks (bigemm_bwd_f32.hip).
 int bwd_gather_f32(const float* x, const float* dy, const float* rscale, const int32_t* tok, const int32_t* chan,

@@ -1,0 +1,65 @@
+// fp32 operands on the bf16 matrix cores: every fp32 value is the sum of three bf16 values
+// (v = v0 + v1 + v2, each the nearest bf16 of what is left: 3 x 8 significand bits, so a value
+// is held to its 24 bits), and a product of two such operands is the six bf16 products whose
+// weight is above 2^-24:
+//     a b = a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0)      (fp32 accumulation)
+// What is left out (a1 b2, a2 b1, a2 b2) is below 2^-25 of the product.  The bf16 MFMAs have 16
+// times the rate of the fp32 ones, so six of them cost 0.375 of one fp32 product.
+#pragma once
+
+#include "ow_device.h"
+
+namespace ow {
+
+// One operand of a 32x32x16 product (8 values per lane) as its three bf16 parts.
+struct X3 {
+  u32x4 p[3];
+};
+
+__device__ __forceinline__ X3 x3_zero() {
+  const u32x4 z = {0u, 0u, 0u, 0u};
+  return X3{{z, z, z}};
+}
+
+// Two fp32 values -> their three parts, packed (first value in the low half).
+__device__ __forceinline__ void x3_split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
+  p0 = BF16::pack2(a, b);
+  const float a1 = a - __uint_as_float(p0 << 16), b1 = b - __uint_as_float(p0 & 0xffff0000u);
+  p1 = BF16::pack2(a1, b1);
+  p2 = BF16::pack2(a1 - __uint_as_float(p1 << 16), b1 - __uint_as_float(p1 & 0xffff0000u));
+}
+
+template <class V>
+__device__ __forceinline__ X3 x3_split8(V v) {  // v(j), j = 0..7
+  X3 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t a, b, c;
+    x3_split2(v(2 * q), v(2 * q + 1), a, b, c);
+    r.p[0][q] = a;
+    r.p[1][q] = b;
+    r.p[2][q] = c;
+  }
+  return r;
+}
+
+// Accumulator registers 8s..8s+7 as an operand (K step s of the next product).
+__device__ __forceinline__ X3 x3_kstep(const f32x16& acc, int s) {
+  return x3_split8([&](int j) { return acc[8 * s + j]; });
+}
+
+__device__ __forceinline__ X3 x3_keep_if(bool keep, const X3& v) {
+  return X3{{keep_if(keep, v.p[0]), keep_if(keep, v.p[1]), keep_if(keep, v.p[2])}};
+}
+
+// c + a b, smallest products first.
+__device__ __forceinline__ f32x16 x3_mma(const X3& a, const X3& b, f32x16 c) {
+  c = BF16::mma32(a.p[2], b.p[0], c);
+  c = BF16::mma32(a.p[1], b.p[1], c);
+  c = BF16::mma32(a.p[0], b.p[2], c);
+  c = BF16::mma32(a.p[1], b.p[0], c);
+  c = BF16::mma32(a.p[0], b.p[1], c);
+  return BF16::mma32(a.p[0], b.p[0], c);
+}
+
+}  // namespace ow

@@ -105,6 +105,13 @@ def pack_weights(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_
     B_u / B_v rows, as OW_FUSE_NORM expects; pad channels are packed as zero.  ``fp8`` packs
     B_u'' / B_v'' as e4m3fn with per-tensor scales (``ow_pack_weights_fp8``) for OW_FUSE_FP8.
     """
+    return _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, norm_weight, plan, gamma, "fp8" if fp8 else "")
+
+
+def _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_weight: Tensor | None,
+          plan: RoutePlan | None, gamma: Tensor | None, layout: str) -> Tensor:
+    """``pack_weights`` in a layout: "" (the compute dtype's own), "fp8", or "x3", three bf16 parts
+    per weight for fp32 activations on the bf16 matrix cores (``ow_pack_weights_x3``)."""
     lib = _native.lib()
     ws = [a_u, a_v, a_o, b_u, b_v, b_o]
     wdtype = ws[0].dtype
@@ -117,7 +124,9 @@ def pack_weights(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_
         raise ValueError("inconsistent BiGEMM weight shapes: "
                          f"a_u {tuple(a_u.shape)}, b_u {tuple(b_u.shape)}, b_v {tuple(b_v.shape)}, b_o {tuple(b_o.shape)}")
     cdt = _DTYPE_CODE[compute_dtype]
-    nbytes = lib.ow_packed_weight_bytes_fp8(q_c, d, rd) if fp8 else lib.ow_packed_weight_bytes(q_c, d, rd, cdt)
+    suffix = f"_{layout}" if layout else ""
+    size, pack = getattr(lib, f"ow_packed_weight_bytes{suffix}"), getattr(lib, f"ow_pack_weights{suffix}")
+    nbytes = size(q_c, d, rd) if layout else size(q_c, d, rd, cdt)
     if nbytes == 0:
         raise ValueError(f"unsupported packing shape q_c={q_c}, d={d}, rd={rd}")
     packed = torch.empty(nbytes, dtype=torch.uint8, device=b_u.device)
@@ -135,14 +144,20 @@ def pack_weights(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_
         if gamma is not None:
             keep.append(gamma.detach().to(device=b_u.device, dtype=torch.float32).contiguous())
             gm_ptr = keep[-1].data_ptr()
-    pack = lib.ow_pack_weights_fp8 if fp8 else lib.ow_pack_weights
+    cdt_arg = () if layout == "x3" else (cdt,)
     with torch.cuda.device(b_u.device):
         _native.check(
             pack(*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype], nw_ptr, gm_ptr, ch_ptr, channels,
-                 SPATIAL_TILE, q_c, d, rd, cdt, packed.data_ptr(), _stream_ptr(b_u.device)),
-            "ow_pack_weights_fp8" if fp8 else "ow_pack_weights",
+                 SPATIAL_TILE, q_c, d, rd, *cdt_arg, packed.data_ptr(), _stream_ptr(b_u.device)),
+            f"ow_pack_weights{suffix}",
         )
     return packed
+
+
+def _x3_supported(plan) -> bool:
+    """Whether fp32 activations of ``plan`` take the matrix-core kernel (``OW_WEIGHTS_X3``): all but
+    images of half a GiB."""
+    return bool(_native.lib().ow_weights_x3_supported(ctypes.byref(native_plan(plan))))
 
 
 def _cached_operands(norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, plan: RoutePlan,
@@ -158,7 +173,8 @@ def _cached_operands(norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, compute_d
     entry = _PackEntry()
     entry.refs = tuple(weakref.ref(t) for t in srcs)
     entry.versions = versions
-    entry.packed = pack_weights(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, norm_weight, plan, gamma, fp8)
+    layout = "fp8" if fp8 else "x3" if compute_dtype == torch.float32 and _x3_supported(plan) else ""
+    entry.packed = _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, norm_weight, plan, gamma, layout)
     if None not in versions:
         _PACK_CACHE[key] = entry
         while len(_PACK_CACHE) > _PACK_CACHE_SIZE:
@@ -225,6 +241,8 @@ def bigemm_fwd(
     lib = _native.lib()
     ws_bytes = lib.ow_fwd_workspace_bytes(ctypes.byref(oplan), x.shape[0], flags)
     workspace = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=x.device)
+    if x.dtype == torch.float32 and _x3_supported(plan):
+        flags |= _native.OW_WEIGHTS_X3  # the layout _cached_operands packs for fp32
     common = (x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(), tok.data_ptr(), ch.data_ptr(),
               ctypes.byref(oplan), x.shape[0], b_u.shape[2], _DTYPE_CODE[x.dtype], flags)
     n_rows = x.shape[0] * plan.height * plan.width

@@ -253,3 +253,23 @@ def test_noalloc_rejects_more_rows_than_the_scratch() -> None:
     rc = lib.ow_bigemm_fwd_noalloc(fake, ctypes.c_void_p(1 << 20), 1e-6, ctypes.c_void_p(1 << 24), nbytes, fake, fake,
                                    ctypes.byref(oplan), b, 2 * d, _native.OW_DTYPE_BF16, flags, None)
     assert rc == 2 and b"scratch" in lib.ow_last_error()
+
+
+def test_x3_weights_refusals_without_touching_the_gpu() -> None:
+    """The three-part fp32 weights: their size, the plans that take them, and what is refused."""
+    lib = _native.lib()
+    assert lib.ow_packed_weight_bytes_x3(4, 128, 256) == 4 * 768 + 4 * 3 * 128 * 256 * 6
+    assert lib.ow_packed_weight_bytes_x3(0, 128, 256) == 0 and lib.ow_packed_weight_bytes_x3(1, 96, 256) == 0
+    plan = _native.make_plan(14, 14, 512, 16, 128, "local", 0)
+    assert lib.ow_weights_x3_supported(ctypes.byref(plan)) == 1
+    huge = _native.make_plan(1024, 1024, 128, 16, 128, "local", 0)  # two images of half a GiB
+    assert lib.ow_weights_x3_supported(ctypes.byref(huge)) == 0
+    P, out = ctypes.c_void_p(16), ctypes.c_void_p(32)
+    nb = lib.ow_packed_weight_bytes_x3(4, 128, 256)
+
+    def fwd(nbytes, dtype):
+        return lib.ow_bigemm_fwd(P, out, 1e-6, P, nbytes, P, P, ctypes.byref(plan), 1, 256, dtype,
+                                 _native.OW_WEIGHTS_X3, None, 0, None)
+
+    assert fwd(nb, _native.OW_DTYPE_BF16) == 2 and b"OW_WEIGHTS_X3" in lib.ow_last_error()
+    assert fwd(nb - 2, _native.OW_DTYPE_F32) == 1 and b"packed weights" in lib.ow_last_error()
