@@ -1,5 +1,4 @@
-// fp32 backward building blocks: the same steps as bigemm_bwd.hip for fp32 activations, as
-// plain one-element-per-thread kernels (fp32 FMAs; no MFMA or vector packing).  The C-ABI
+// fp32 backward building blocks: the same steps as bigemm_bwd.hip for fp32 activations.  The C-ABI
 // launchers of bigemm_bwd.hip call these when dtype is OW_DTYPE_F32.
 #include <hip/hip_runtime.h>
 
@@ -75,26 +74,35 @@ __global__ void __launch_bounds__(256) scatter_f32_kernel(const float* dxt, cons
   if (row >= 0 && ch >= 0 && ch < channels) g[row * channels + ch] = dxt[i];
 }
 
-__global__ void __launch_bounds__(256) rmsnorm_bwd_f32_kernel(const float* x, const float* g, const float* rscale,
-                                                              const float* dout, float* dx, int64_t rows,
-                                                              int32_t channels, int32_t residual) {
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= rows) return;
-  const float* xr = x + row * channels;
-  const float* gr = g + row * channels;
+// dx = (dout) + r g - x r^3 / C sum_c(g x), one row per LPR lanes of 4 channels each (C % 4 == 0,
+// 16-byte aligned rows, VEC), or one per wave with one channel per lane step.
+template <int LPR, bool VEC>
+__global__ void __launch_bounds__(256) rmsnorm_bwd_f32_kernel(const float* __restrict__ x, const float* __restrict__ g,
+                                                              const float* __restrict__ rscale,
+                                                              const float* __restrict__ dout, float* __restrict__ dx,
+                                                              int64_t rows, int32_t channels, int32_t residual) {
+  constexpr int RPB = 256 / LPR, W = VEC ? 4 : 1;
+  typedef float vec __attribute__((ext_vector_type(W)));
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + threadIdx.x / LPR;
+  const int sub = threadIdx.x % LPR;
+  if (row >= rows) return;  // whole groups of LPR lanes leave together
+  auto at = [&](const float* p, int c) { return *reinterpret_cast<const vec*>(p + row * channels + c); };
   float r = 1.0f, coef = 0.0f;
   if (rscale) {
     r = rscale[row];
     float dot = 0.0f;
-    for (int c = lane; c < channels; c += 64) dot = fmaf(gr[c], xr[c], dot);
-    for (int m = 32; m > 0; m >>= 1) dot += __shfl_xor(dot, m);
+    for (int c = W * sub; c < channels; c += W * LPR) {
+      const vec xv = at(x, c), gv = at(g, c);
+#pragma unroll
+      for (int k = 0; k < W; ++k) dot = fmaf(gv[k], xv[k], dot);
+    }
+    for (int m = LPR / 2; m > 0; m >>= 1) dot += __shfl_xor(dot, m);
     coef = dot * r * r * r / static_cast<float>(channels);
   }
-  for (int c = lane; c < channels; c += 64) {
-    float v = r * gr[c] - coef * xr[c];
-    if (residual) v += dout[row * channels + c];
-    dx[row * channels + c] = v;
+  for (int c = W * sub; c < channels; c += W * LPR) {
+    vec v = r * at(g, c) - coef * at(x, c);
+    if (residual) v += at(dout, c);
+    *reinterpret_cast<vec*>(dx + row * channels + c) = v;
   }
 }
 
@@ -138,46 +146,99 @@ __global__ void __launch_bounds__(256) fold_f32_kernel(FoldF32Args a, int64_t to
   a.boT[cd] = o;
 }
 
-// out[t][i][c] = sum_j M1[i][j] in1[t][j][c] (+ M2[i][j] in2[t][j][c]).
-__global__ void __launch_bounds__(256) tile_mix_f32_kernel(const float* in1, const float* m1, const float* in2,
-                                                           const float* m2, float* out, int64_t total, int32_t d) {
+// out[t][i][c] = sum_j M1[i][j] in1[t][j][c] (+ M2[i][j] in2[t][j][c]): one thread per (tile,
+// column) holds the column's 16 values and forms its 16 outputs, the matrices from scalar
+// registers, so each value is read once (a thread per output read it 16 times).  Bound by
+// memory: 25,088 slots x 4 groups x 64 channels, one input, 33 -> 10.5 us.
+template <bool TWO>
+__global__ void __launch_bounds__(256) tile_mix_f32_kernel(const float* __restrict__ in1, const float* __restrict__ m1,
+                                                           const float* __restrict__ in2, const float* __restrict__ m2,
+                                                           float* __restrict__ out, int64_t columns, int32_t d) {
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const int32_t c = static_cast<int32_t>(idx % d);
-  const int32_t i = static_cast<int32_t>((idx / d) % kG);
-  const int64_t base = (idx / (static_cast<int64_t>(kG) * d)) * kG * d + c;
-  float acc = 0.0f;
+  if (idx >= columns) return;
+  const int64_t tile = idx / d;
+  const int64_t base = tile * kG * d + (idx - tile * d);
+  float v[kG], w[TWO ? kG : 1];
 #pragma unroll
-  for (int j = 0; j < kG; ++j) acc = fmaf(m1[i * kG + j], in1[base + static_cast<int64_t>(j) * d], acc);
-  if (in2) {
+  for (int j = 0; j < kG; ++j) v[j] = in1[base + static_cast<int64_t>(j) * d];
+  if constexpr (TWO) {
 #pragma unroll
-    for (int j = 0; j < kG; ++j) acc = fmaf(m2[i * kG + j], in2[base + static_cast<int64_t>(j) * d], acc);
+    for (int j = 0; j < kG; ++j) w[j] = in2[base + static_cast<int64_t>(j) * d];
   }
-  out[idx] = acc;
+#pragma unroll
+  for (int i = 0; i < kG; ++i) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kG; ++j) acc = fmaf(m1[i * kG + j], v[j], acc);
+    if constexpr (TWO) {
+#pragma unroll
+      for (int j = 0; j < kG; ++j) acc = fmaf(m2[i * kG + j], w[j], acc);
+    }
+    out[base + static_cast<int64_t>(i) * d] = acc;
+  }
 }
 
-// partial[i][j][w] = sum over tiles t = w, w + n_waves, ... of sum_c in1[t][i][c] in2[t][j][c];
-// lane l of wave w owns outputs 4l .. 4l + 3.
-__global__ void __launch_bounds__(256) tile_outer_f32_kernel(const float* in1, const float* in2, float* partial,
-                                                             int64_t n_tiles, int32_t d) {
-  const int lane = threadIdx.x & 63;
+// partial[i][j][w] = sum over tiles t = w, w + n_waves, ... of sum_c in1[t][i][c] in2[t][j][c]
+// on the fp32 16x16x4 MFMA: lane (row l16, h) holds channels 16 s + 4 h .. + 3 of its row, and
+// product j of a 16-channel step takes component j of both operands.  Bound by memory (each tile
+// is read once, 64-byte pieces of 16 rows per instruction), so with few waves the loads of two
+// tiles are in flight before the first product (D, the compile-time d; 0: any, one step at a
+// time).  The same shape took 169 us with one serial dot product per output, 18 us now.
+template <bool VEC, int D>
+__global__ void __launch_bounds__(256) tile_outer_f32_kernel(const float* __restrict__ in1, const float* __restrict__ in2,
+                                                             float* __restrict__ partial, int64_t n_tiles, int32_t d) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, h = lane >> 4;
   const int64_t wave = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * 4;
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int64_t t = wave; t < n_tiles; t += n_waves) {
-    const int64_t base = t * kG * d;
+  auto load = [&](const float* p) {
+    if constexpr (VEC) {
+      return *reinterpret_cast<const f32x4*>(p);
+    } else {
+      return f32x4{p[0], p[1], p[2], p[3]};
+    }
+  };
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 acc = zero;  // sum over tiles; a tile's own sum is formed apart, so the fp32 chains stay short
+  auto mma = [&](const f32x4& a, const f32x4& b, f32x4& c) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int o = 4 * lane + k, i = o / kG, j = o % kG;
-      const float* a = in1 + base + static_cast<int64_t>(i) * d;
-      const float* b = in2 + base + static_cast<int64_t>(j) * d;
-      float s = 0.0f;
-      for (int c = 0; c < d; ++c) s = fmaf(a[c], b[c], s);
-      acc[k] += s;
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+  };
+  if constexpr (D > 0) {
+    constexpr int N = D / 16;
+    for (int64_t t = wave; t < n_tiles; t += 2 * n_waves) {
+      const bool two = t + n_waves < n_tiles;
+      const int64_t b0 = (t * kG + l16) * D + 4 * h, b1 = ((two ? t + n_waves : t) * kG + l16) * D + 4 * h;
+      f32x4 u[2][N], v[2][N];
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        u[0][c] = load(in1 + b0 + 16 * c);
+        v[0][c] = load(in2 + b0 + 16 * c);
+      }
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        u[1][c] = load(in1 + b1 + 16 * c);
+        v[1][c] = load(in2 + b1 + 16 * c);
+      }
+      f32x4 s[2] = {zero, zero};
+#pragma unroll
+      for (int c = 0; c < N; ++c) {
+        mma(u[0][c], v[0][c], s[0]);
+        mma(u[1][c], v[1][c], s[1]);
+      }
+      mfma_drain();
+      acc += two ? s[0] + s[1] : s[0];
+    }
+  } else {
+    for (int64_t t = wave; t < n_tiles; t += n_waves) {
+      const int64_t base = (t * kG + l16) * d + 4 * h;
+      f32x4 s = zero;
+      for (int c = 0; c < d; c += 16) mma(load(in1 + base + c), load(in2 + base + c), s);
+      mfma_drain();
+      acc += s;
     }
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k) partial[(4 * lane + k) * n_waves + wave] = acc[k];
+  for (int k = 0; k < 4; ++k) partial[static_cast<int64_t>((4 * h + k) * kG + l16) * n_waves + wave] = acc[k];
 }
 
 }  // namespace
@@ -207,8 +268,20 @@ int bwd_scatter_f32(const float* dxt, const int32_t* tok, const int32_t* chan, f
 
 int bwd_rmsnorm_f32(const float* x, const float* g, const float* rscale, const float* dout, float* dx, int64_t rows,
                     int32_t channels, int32_t residual, hipStream_t s) {
-  hipLaunchKernelGGL(rmsnorm_bwd_f32_kernel, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, s, x, g,
-                     rscale, dout, dx, rows, channels, residual);
+  auto launch = [&](auto lpr, auto vec) {
+    constexpr int L = decltype(lpr)::value;
+    hipLaunchKernelGGL((rmsnorm_bwd_f32_kernel<L, decltype(vec)::value>),
+                       dim3(static_cast<unsigned>((rows * L + 255) / 256)), dim3(256), 0, s, x, g, rscale, dout, dx, rows,
+                       channels, residual);
+  };
+  const std::integral_constant<bool, true> vec;
+  const bool aligned = channels % 4 == 0 && aligned16(x) && aligned16(g) && aligned16(dx) && (!residual || aligned16(dout));
+  if (!aligned)
+    launch(std::integral_constant<int, 64>{}, std::integral_constant<bool, false>{});
+  else if (channels <= 128)  // a row in one step of half a wave
+    launch(std::integral_constant<int, 32>{}, vec);
+  else
+    launch(std::integral_constant<int, 64>{}, vec);
   return hip_status(hipGetLastError(), "rmsnorm_bwd_f32_kernel launch");
 }
 
@@ -223,15 +296,26 @@ int fold_weights_f32(const void* b_u, const void* b_v, const void* b_o, int32_t 
 
 int tile_mix_f32(const float* in1, const float* m1, const float* in2, const float* m2, float* out, int64_t n_tiles,
                  int32_t d, hipStream_t s) {
-  const int64_t total = n_tiles * kG * d;
-  hipLaunchKernelGGL(tile_mix_f32_kernel, dim3(grid_for(total)), dim3(256), 0, s, in1, m1, in2, m2, out, total, d);
+  const int64_t columns = n_tiles * d;
+  if (in2)
+    hipLaunchKernelGGL(tile_mix_f32_kernel<true>, dim3(grid_for(columns)), dim3(256), 0, s, in1, m1, in2, m2, out,
+                       columns, d);
+  else
+    hipLaunchKernelGGL(tile_mix_f32_kernel<false>, dim3(grid_for(columns)), dim3(256), 0, s, in1, m1, in2, m2, out,
+                       columns, d);
   return hip_status(hipGetLastError(), "tile_mix_f32_kernel launch");
 }
 
 int tile_outer_f32(const float* in1, const float* in2, float* partial, int32_t n_waves, int64_t n_tiles, int32_t d,
                    hipStream_t s) {
-  hipLaunchKernelGGL(tile_outer_f32_kernel, dim3(static_cast<unsigned>(n_waves / 4)), dim3(256), 0, s, in1, in2,
-                     partial, n_tiles, d);
+  const dim3 grid(static_cast<unsigned>(n_waves / 4));
+  const bool vec = aligned16(in1) && aligned16(in2);
+  if (vec && d == 64)
+    hipLaunchKernelGGL((tile_outer_f32_kernel<true, 64>), grid, dim3(256), 0, s, in1, in2, partial, n_tiles, d);
+  else if (vec && d == 128)
+    hipLaunchKernelGGL((tile_outer_f32_kernel<true, 128>), grid, dim3(256), 0, s, in1, in2, partial, n_tiles, d);
+  else
+    hipLaunchKernelGGL((tile_outer_f32_kernel<false, 0>), grid, dim3(256), 0, s, in1, in2, partial, n_tiles, d);
   return hip_status(hipGetLastError(), "tile_outer_f32_kernel launch");
 }
 
