@@ -490,6 +490,30 @@ int ow_bwd_params(const void* b_u, const void* b_v, const void* b_o, int32_t wei
 int ow_small_to_f32(const void* const* src, const int32_t* dtype, const int64_t* count, int32_t n, float* dst,
                     void* stream);
 
+/*
+ * The whole bf16 / fp16 backward of a block as one call (the reference's autograd recompute,
+ * omniweave/ops/triton.py:256-292), for d = 128 and for d = 64 with batch * Q_s even:
+ * ow_bwd_block_workspace returns the bytes it needs (drop, scales: whether drop_scale and
+ * row_scale will be given), or 0 when the shape or dtype has no such path and the caller composes
+ * the entry points above (fp32, d = 64 with an odd number of token groups).
+ *   grad, x      [B, H*W, C] of dtype; small: norm weight (NULL without OW_FUSE_NORM), gamma,
+ *                A_u, A_v, A_o with their dtypes; b_u, b_v, b_o of weight_dtype, contiguous
+ *   row_scale    the forward's RMSNorm scales (ow_bigemm_fwd_scales), or NULL: formed here
+ *   drop_scale   [B] per-image factors of the forward, or NULL
+ *   dx           [B, H*W, C] of dtype
+ *   grads        fp32: dA_u, dA_v, dA_o (256 each), dB_u, dB_v, dB_o, dgamma and, with the norm,
+ *                dnorm_weight; 16-byte aligned
+ *   cast         NULL, or the same values in cast_dtype (bf16 / fp16), 8-byte aligned
+ *   workspace    16-byte aligned
+ */
+size_t ow_bwd_block_workspace(const OwPlan* plan, int32_t batch, int32_t rd, int32_t dtype, int32_t flags,
+                              int32_t drop, int32_t scales);
+int ow_bwd_block(const void* grad, const void* x, const void* const* small, const int32_t* small_dtype,
+                 const void* b_u, const void* b_v, const void* b_o, int32_t weight_dtype, const float* row_scale,
+                 const float* drop_scale, const int32_t* token_index, const int32_t* channel_index,
+                 const OwPlan* plan, int32_t batch, int32_t rd, int32_t dtype, int32_t flags, float eps, void* dx,
+                 float* grads, void* cast, int32_t cast_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

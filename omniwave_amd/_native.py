@@ -42,6 +42,13 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 6 + [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]
         + [ctypes.c_int32] * 5 + [ctypes.c_void_p, ctypes.c_void_p],
     ),
+    "ow_bwd_block_workspace": (ctypes.c_size_t, [ctypes.POINTER(OwPlan)] + [ctypes.c_int32] * 6),
+    "ow_bwd_block": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 7 + [ctypes.c_int32] + [ctypes.c_void_p] * 4
+        + [ctypes.POINTER(OwPlan), ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_float]
+        + [ctypes.c_void_p] * 3 + [ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p],
+    ),
     "ow_weights_x3_supported": (ctypes.c_int32, [ctypes.POINTER(OwPlan)]),
     "ow_packed_weight_bytes_x3": (ctypes.c_size_t, [ctypes.c_int32] * 3),
     "ow_pack_weights_x3": (
@@ -225,6 +232,8 @@ class NativeLibraryError(RuntimeError):
 
 def _load() -> ctypes.CDLL | None:
     global _lib, _load_error
+    if _lib is not None:  # set once, under the lock
+        return _lib
     with _lock:
         if _lib is not None or _load_error is not None:
             return _lib

@@ -4,6 +4,8 @@ Replaces the fp32 autograd recompute of the accelerated backend
 (omniweave/ops/triton.py:256-292).  The pass runs in the forward's compute dtype with fp32
 accumulation, entirely on the HIP stream of the gradient:
 
+* for bf16 / fp16 one native call (``ow_bwd_block``) launches the kernels below in order; fp32 and
+  d = 64 with an odd number of token groups are composed here;
 * routing, RMSNorm, gate and parameter fold-back are the libomniwave_amd.so kernels
   (``ow_bwd_gather``, ``ow_bwd_gate``, ``ow_bwd_scatter``, ``ow_bwd_rmsnorm``,
   ``ow_bwd_params``, ``ow_fold_weights``);
@@ -55,7 +57,7 @@ _SPLITS = 64
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _tile_mix(lib, in1: Tensor, m1: Tensor, in2: Tensor | None, m2: Tensor | None, d: int, code: int,
@@ -129,7 +131,7 @@ def native_batch_limit(dtype: torch.dtype, plan: RoutePlan, q_c: int, d: int, rd
     """
     if dtype == torch.float32:
         return None
-    elt = torch.empty((), dtype=dtype).element_size()
+    elt = dtype.itemsize
     q_s = int(plan.token_indices.shape[0])
     per_image = max(plan.height * plan.width * plan.channels, q_c * q_s * 16 * max(d, rd)) * elt
     return max(1, (_ADDR_LIMIT - 1) // per_image)
@@ -173,14 +175,16 @@ def bigemm_backward(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: 
     if row_scale is not None and row_scale.numel() != x.shape[0] * n_tok:
         row_scale = None
     if len(chunks) == 1:
-        dx, g_all = _backward_once(grad, x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, flags, eps,
-                                   drop_scale, row_scale)
+        dx, g_all, cast = _backward_once(grad, x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, flags, eps,
+                                         drop_scale, row_scale, True)
+        if cast is not None:
+            return (dx, *_grad_views(cast, fuse_norm, plan.channels, q_c, d, rd))
     else:
         dxs, g_all = [], None
         for s, e in chunks:
-            dx_c, g_c = _backward_once(grad[s:e], x[s:e], norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan,
-                                       flags, eps, drop_scale[s:e] if drop_scale is not None else None,
-                                       row_scale[s * n_tok:e * n_tok] if row_scale is not None else None)
+            dx_c, g_c, _ = _backward_once(grad[s:e], x[s:e], norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan,
+                                          flags, eps, drop_scale[s:e] if drop_scale is not None else None,
+                                          row_scale[s * n_tok:e * n_tok] if row_scale is not None else None, False)
             dxs.append(dx_c)
             g_all = g_c if g_all is None else g_all.add_(g_c)
         dx = torch.cat(dxs)
@@ -188,23 +192,23 @@ def bigemm_backward(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: 
                        norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)
 
 
+def _grad_views(buf: Tensor, fuse_norm: bool, channels: int, q_c: int, d: int, rd: int):
+    """The parameter gradients as views of the buffer of ``_cast_grads``."""
+    nb = q_c * d * rd
+    a_u, a_v, a_o, b_u, b_v, b_o, c = torch.split(buf, (256, 256, 256, nb, nb, nb, buf.numel() - 768 - 3 * nb))
+    gamma, norm_weight = torch.split(c, channels) if fuse_norm else (c, None)
+    return (norm_weight, gamma, a_u.view(16, 16), a_v.view(16, 16), a_o.view(16, 16),
+            b_u.view(q_c, d, rd), b_v.view(q_c, d, rd), b_o.view(q_c, rd, d))
+
+
 def _cast_grads(dx, g_all, fuse_norm, channels, q_c, d, rd, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o):
     """Parameter gradients as views of the fp32 buffer ``g_all`` (the token matrices, B_u, B_v,
     B_o, then gamma and the norm weight), cast to each parameter's dtype: one cast of the whole
     buffer when they share a dtype."""
-    nb = q_c * d * rd
     params = ([norm_weight] if fuse_norm else []) + [gamma, a_u, a_v, a_o, b_u, b_v, b_o]
-
-    def views(buf):
-        o_a = buf[:768].view(3, 16, 16)
-        o_b = buf[768:768 + 3 * nb]
-        o_c = buf[768 + 3 * nb:].view(-1, channels)
-        return (o_c[1] if fuse_norm else None, o_c[0], o_a[0], o_a[1], o_a[2],
-                o_b[:nb].view(q_c, d, rd), o_b[nb:2 * nb].view(q_c, d, rd), o_b[2 * nb:].view(q_c, rd, d))
-
     if len({t.dtype for t in params}) == 1:
-        return (dx, *views(g_all.to(params[0].dtype)))
-    g_nw, g_gamma, g_au, g_av, g_ao, g_bu, g_bv, g_bo = views(g_all)
+        return (dx, *_grad_views(g_all.to(params[0].dtype), fuse_norm, channels, q_c, d, rd))
+    g_nw, g_gamma, g_au, g_av, g_ao, g_bu, g_bv, g_bo = _grad_views(g_all, fuse_norm, channels, q_c, d, rd)
     return (
         dx,
         g_nw.to(norm_weight.dtype) if g_nw is not None else None,
@@ -216,9 +220,11 @@ def _cast_grads(dx, g_all, fuse_norm, channels, q_c, d, rd, norm_weight, gamma, 
 
 def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: Tensor, a_u: Tensor, a_v: Tensor,
                    a_o: Tensor, b_u: Tensor, b_v: Tensor, b_o: Tensor, plan: RoutePlan, flags: int, eps: float,
-                   drop_scale: Tensor | None, row_scale: Tensor | None = None):
-    """One pass of the kernels over the whole batch: dx and the fp32 parameter-gradient buffer
-    (layout of ``_cast_grads``)."""
+                   drop_scale: Tensor | None, row_scale: Tensor | None, want_cast: bool):
+    """One pass of the kernels over the whole batch: dx, the fp32 parameter-gradient buffer (layout
+    of ``_cast_grads``) and, with ``want_cast`` and parameters of one 16-bit dtype, that buffer in
+    their dtype (else None).  bf16 / fp16 shapes with kernels of their own run as one native call
+    (``ow_bwd_block``); the rest is composed here."""
     lib = _native.lib()
     dev = x.device
     dtype = x.dtype
@@ -226,7 +232,8 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
     fuse_norm = bool(flags & _native.OW_FUSE_NORM)
     residual = bool(flags & _native.OW_FUSE_RESIDUAL)
     x = x.contiguous()
-    grad = grad.to(dtype).contiguous()
+    if grad.dtype != dtype or not grad.is_contiguous():
+        grad = grad.to(dtype).contiguous()
     batch = x.shape[0]
     q_c, d, rd = b_u.shape
     q_s = plan.token_indices.shape[0]
@@ -237,11 +244,36 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
     stream = _stream(dev)
     grad_delta = grad  # upstream gradient of the delta branch (drop-path scaled below)
 
-    ws = [w.detach().contiguous() for w in (b_u, b_v, b_o)]
+    ws = [w if w.is_contiguous() else w.detach().contiguous() for w in (b_u, b_v, b_o)]
     wdtype = ws[0].dtype
     if any(w.dtype != wdtype for w in ws) or wdtype not in _DTYPE_CODE:
         wdtype = torch.float32
-        ws = [w.float() for w in ws]
+        ws = [w.detach().float() for w in ws]
+    nbytes = lib.ow_bwd_block_workspace(ctypes.byref(oplan), batch, rd, code, flags, drop_scale is not None,
+                                        row_scale is not None)
+    if nbytes:
+        small = [(t if t.is_contiguous() else t.contiguous()) if t.device == dev and t.dtype in _DTYPE_CODE
+                 else _fp32(t, dev) for t in (norm_weight if fuse_norm else gamma, gamma, a_u, a_v, a_o)]
+        n = 768 + 3 * q_c * d * rd + (2 if fuse_norm else 1) * plan.channels
+        g_all = torch.empty(n, dtype=torch.float32, device=dev)
+        dts = {t.dtype for t in ((norm_weight,) if fuse_norm else ()) + (gamma, a_u, a_v, a_o, b_u, b_v, b_o)}
+        cast_dtype = dts.pop() if len(dts) == 1 else None
+        cast = (torch.empty(n, dtype=cast_dtype, device=dev)
+                if want_cast and cast_dtype in (torch.bfloat16, torch.float16) else None)
+        scale = drop_scale.to(device=dev, dtype=torch.float32).contiguous() if drop_scale is not None else None
+        rscale = row_scale.to(device=dev, dtype=torch.float32).contiguous() if row_scale is not None else None
+        dx = torch.empty_like(x)
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            _native.check(lib.ow_bwd_block(
+                grad.data_ptr(), x.data_ptr(), (ctypes.c_void_p * 5)(*[t.data_ptr() for t in small]),
+                (ctypes.c_int32 * 5)(*[_DTYPE_CODE[t.dtype] for t in small]), ws[0].data_ptr(), ws[1].data_ptr(),
+                ws[2].data_ptr(), _DTYPE_CODE[wdtype], rscale.data_ptr() if rscale is not None else None,
+                scale.data_ptr() if scale is not None else None, tok.data_ptr(), ch.data_ptr(), ctypes.byref(oplan), batch,
+                rd, code, flags, eps, dx.data_ptr(), g_all.data_ptr(), cast.data_ptr() if cast is not None else None,
+                _DTYPE_CODE[cast_dtype] if cast is not None else 0, workspace.data_ptr(), nbytes, stream), "ow_bwd_block")
+        return dx, g_all, cast
+
     # The small fp32 operands (norm weight, gamma, token matrices): one conversion kernel into
     # one buffer (ow_small_to_f32).
     small = ([norm_weight] if fuse_norm else []) + [gamma, a_u, a_v, a_o]
@@ -283,165 +315,55 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
             _native.check(lib.ow_rms_scale(x.data_ptr(), rscale.data_ptr(), n_rows, plan.channels, eps, code,
                                            stream), "ow_rms_scale")
 
-        fused = d == 64 and slots % 32 == 0 and dtype != torch.float32
-        chan128 = d == 128 and dtype != torch.float32
-        # The d = 64 fused kernel and the d = 128 channel kernels read x / dy and write g
-        # themselves when group q is channels [d q, d q + d) (routing.py:107-121: radix level 0
-        # or a single group): no gather and no scatter pass.
-        identity = plan.channels == q_c * d and (plan.radix_level == 0 or q_c == 1)
-        routed = (fused or chan128) and identity
         g = torch.empty(n_rows, plan.channels, dtype=dtype, device=dev)  # fully written: no clearing
-        rs_ptr = rscale.data_ptr() if rscale is not None else None
-        if not routed:
-            # Routed tiles of X' = x r and of dY.
-            xt = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
-            dyt = torch.empty_like(xt)
-            _native.check(lib.ow_bwd_gather(x.data_ptr(), grad_delta.data_ptr(), rscale.data_ptr() if rscale is not None
-                                            else None, tok.data_ptr(), ch.data_ptr(), ctypes.byref(oplan),
-                                            batch, code, xt.data_ptr(), dyt.data_ptr(), stream), "ow_bwd_gather")
+        # Routed tiles of X' = x r and of dY.
+        xt = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
+        dyt = torch.empty_like(xt)
+        _native.check(lib.ow_bwd_gather(x.data_ptr(), grad_delta.data_ptr(), rscale.data_ptr() if rscale is not None
+                                        else None, tok.data_ptr(), ch.data_ptr(), ctypes.byref(oplan),
+                                        batch, code, xt.data_ptr(), dyt.data_ptr(), stream), "ow_bwd_gather")
+        # Folded weights in the compute dtype, plain and transposed (both contiguous).
+        bu = torch.empty(q_c, d, rd, dtype=dtype, device=dev)
+        bv, bo_t = torch.empty_like(bu), torch.empty_like(bu)
+        bu_t = torch.empty(q_c, rd, d, dtype=dtype, device=dev)
+        bv_t, bo = torch.empty_like(bu_t), torch.empty_like(bu_t)
+        _native.check(lib.ow_fold_weights(*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype],
+                                          nw.data_ptr() if nw is not None else None, gm.data_ptr(), ch.data_ptr(),
+                                          plan.channels, q_c, d, rd, code, bu.data_ptr(), bu_t.data_ptr(),
+                                          bv.data_ptr(), bv_t.data_ptr(), bo.data_ptr(), bo_t.data_ptr(), stream),
+                      "ow_fold_weights")
+        au_t, av_t, ao_t = (a.t().contiguous() for a in (au, av, ao))
+        # Token side: P_u = A_u X', P_v = A_v X', dW' = A_o^T dY (per 16-slot tile).
+        pu = _tile_mix(lib, xt, au, None, None, d, code, stream)
+        pv = _tile_mix(lib, xt, av, None, None, d, code, stream)
+        dw = _tile_mix(lib, dyt, ao_t, None, None, d, code, stream)
+        # Channel side: batched GEMMs + the gate kernel.
+        u = torch.bmm(pu, bu)
+        v = torch.bmm(pv, bv)
+        dz = torch.bmm(dw, bo_t)
+        z, du, dv = torch.empty_like(u), torch.empty_like(u), torch.empty_like(u)
+        _native.check(lib.ow_bwd_gate(u.data_ptr(), v.data_ptr(), dz.data_ptr(), z.data_ptr(), du.data_ptr(),
+                                      dv.data_ptr(), u.numel(), code, stream), "ow_bwd_gate")
+        del u, v, dz
+        wp = torch.bmm(z, bo)
+        dpu = torch.bmm(du, bu_t)
+        dpv = torch.bmm(dv, bv_t)
+        d_bu = _slot_reduce(pu, du)   # [q_c, d, rd]
+        d_bv = _slot_reduce(pv, dv)
+        d_bo = _slot_reduce(z, dw)    # [q_c, rd, d]
+        del z, du, dv, pu, pv, dw
 
-        if fused:
-            # One fused kernel: token side, channel side and gate, dX', and the token-matrix
-            # gradients as per-workgroup partials.
-            nbytes = lib.ow_bwd_packed_bytes(q_c, d, rd)
-            wpk = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            _native.check(lib.ow_pack_bwd_weights(*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype],
-                                                  nw.data_ptr() if nw is not None else None, gm.data_ptr(),
-                                                  ch.data_ptr(), plan.channels, q_c, d, rd, code, wpk.data_ptr(),
-                                                  stream), "ow_pack_bwd_weights")
-            pu = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
-            pv, dw = torch.empty_like(pu), torch.empty_like(pu)
-            n_part = lib.ow_bwd_fused_partials(slots, q_c, rd)
-            partial = torch.empty(n_part, 3, 256, dtype=torch.float32, device=dev)
-            if routed:
-                _native.check(lib.ow_bwd_fused_routed(x.data_ptr(), grad_delta.data_ptr(), rscale.data_ptr() if rscale
-                                                      is not None else None, tok.data_ptr(),
-                                                      ctypes.byref(oplan), batch, au.data_ptr(),
-                                                      av.data_ptr(), ao.data_ptr(), wpk.data_ptr(), nbytes,
-                                                      pu.data_ptr(), pv.data_ptr(), dw.data_ptr(), g.data_ptr(),
-                                                      partial.data_ptr(), n_part, rd, code, stream),
-                              "ow_bwd_fused_routed")
-            else:
-                dxt = torch.empty_like(xt)
-                _native.check(lib.ow_bwd_fused(xt.data_ptr(), dyt.data_ptr(), au.data_ptr(), av.data_ptr(),
-                                               ao.data_ptr(), wpk.data_ptr(), nbytes, pu.data_ptr(), pv.data_ptr(),
-                                               dw.data_ptr(), dxt.data_ptr(), partial.data_ptr(), n_part, slots, q_c,
-                                               d, rd, code, stream), "ow_bwd_fused")
-                del xt, dyt
-            _sum_rows(lib, partial, n_part, g_a, stream)  # [3, 256]: dA_u, dA_v, dA_o
-            g_au, g_av, g_ao = (g_a[m].view(16, 16) for m in range(3))
-            # dB_u'', dB_v'', dB_o'' from P_u, P_v, dW' (the gate recomputed): per slot range one
-            # [3, q_c, d * rd] block, summed over the ranges.
-            n_red = lib.ow_bwd_param_reduce64_partials(slots, q_c, rd)
-            red = torch.empty(n_red, 3 * d * rd, dtype=torch.float32, device=dev)
-            _native.check(lib.ow_bwd_param_reduce64(pu.data_ptr(), pv.data_ptr(), dw.data_ptr(), wpk.data_ptr(), nbytes,
-                                                    red.data_ptr(), n_red, slots, q_c, rd, code, stream),
-                          "ow_bwd_param_reduce64")
-            g_b3 = torch.empty(3, q_c, d * rd, dtype=torch.float32, device=dev)
-            _sum_rows(lib, red, n_red // q_c, g_b3, stream)
-            d_bu = g_b3[0].view(q_c, d, rd)
-            d_bv = g_b3[1].view(q_c, d, rd)
-            d_bo = g_b3[2].view(q_c, rd, d)
-            del pu, pv, dw
-        elif d == 128 and dtype != torch.float32:
-            # Two kernels over 256-slot units: (1) token side P_u, P_v, dW', then U', V', dZ per
-            # 32-row chunk and the gate backward (Z, dU', dV'); (2) dP_u, dP_v, dX', W' and the
-            # token-matrix gradients (per-workgroup partials).
-            nbytes = lib.ow_bwd_packed_bytes(q_c, d, rd)
-            wpk = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            _native.check(lib.ow_pack_bwd_weights(*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype],
-                                                  nw.data_ptr() if nw is not None else None, gm.data_ptr(),
-                                                  ch.data_ptr(), plan.channels, q_c, d, rd, code, wpk.data_ptr(),
-                                                  stream), "ow_pack_bwd_weights")
-            pu = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
-            pv, dw = torch.empty_like(pu), torch.empty_like(pu)
-            z = torch.empty(q_c, slots, rd, dtype=dtype, device=dev)
-            du, dv = torch.empty_like(z), torch.empty_like(z)
-            n_part = lib.ow_bwd_channel_partials(slots, q_c)
-            partial = torch.empty(n_part, 3, 256, dtype=torch.float32, device=dev)
-            if routed:
-                _native.check(lib.ow_bwd_channel_routed(x.data_ptr(), grad_delta.data_ptr(), rs_ptr, tok.data_ptr(),
-                                                        ctypes.byref(oplan), batch, au.data_ptr(), av.data_ptr(),
-                                                        ao.data_ptr(), wpk.data_ptr(), nbytes, pu.data_ptr(),
-                                                        pv.data_ptr(), dw.data_ptr(), z.data_ptr(), du.data_ptr(),
-                                                        dv.data_ptr(), rd, code, stream), "ow_bwd_channel_routed")
-                _native.check(lib.ow_bwd_channel2_routed(x.data_ptr(), grad_delta.data_ptr(), rs_ptr, z.data_ptr(),
-                                                         du.data_ptr(), dv.data_ptr(), au.data_ptr(), av.data_ptr(),
-                                                         wpk.data_ptr(), nbytes, tok.data_ptr(), ctypes.byref(oplan),
-                                                         batch, g.data_ptr(), partial.data_ptr(), n_part, rd, code,
-                                                         stream), "ow_bwd_channel2_routed")
-            else:
-                _native.check(lib.ow_bwd_channel(xt.data_ptr(), dyt.data_ptr(), au.data_ptr(), av.data_ptr(),
-                                                 ao.data_ptr(), wpk.data_ptr(), nbytes, pu.data_ptr(), pv.data_ptr(),
-                                                 dw.data_ptr(), z.data_ptr(), du.data_ptr(), dv.data_ptr(), slots,
-                                                 q_c, d, rd, code, stream), "ow_bwd_channel")
-                dxt = torch.empty_like(xt)
-                _native.check(lib.ow_bwd_channel2(xt.data_ptr(), dyt.data_ptr(), z.data_ptr(), du.data_ptr(),
-                                                  dv.data_ptr(), au.data_ptr(), av.data_ptr(), wpk.data_ptr(), nbytes,
-                                                  dxt.data_ptr(), partial.data_ptr(), n_part, slots, q_c, d, rd, code,
-                                                  stream), "ow_bwd_channel2")
-            _sum_rows(lib, partial, n_part, g_a, stream)  # [3, 256]: dA_u, dA_v, dA_o
-            g_au, g_av, g_ao = (g_a[m].view(16, 16) for m in range(3))
-            # dB_u'', dB_v'', dB_o'' from the slot-major intermediates, as for d = 64.
-            n_red = lib.ow_bwd_param_reduce128_partials(slots, q_c, rd)
-            red = torch.empty(n_red, 3 * d * rd, dtype=torch.float32, device=dev)
-            _native.check(lib.ow_bwd_param_reduce128(pu.data_ptr(), pv.data_ptr(), dw.data_ptr(), z.data_ptr(),
-                                                     du.data_ptr(), dv.data_ptr(), red.data_ptr(), n_red, slots, q_c,
-                                                     rd, code, stream), "ow_bwd_param_reduce128")
-            g_b3 = torch.empty(3, q_c, d * rd, dtype=torch.float32, device=dev)
-            _sum_rows(lib, red, n_red // q_c, g_b3, stream)
-            d_bu = g_b3[0].view(q_c, d, rd)
-            d_bv = g_b3[1].view(q_c, d, rd)
-            d_bo = g_b3[2].view(q_c, rd, d)
-            del wpk, z, du, dv, pu, pv, dw
-            if not routed:
-                del xt, dyt
-        else:
-            # Folded weights in the compute dtype, plain and transposed (both contiguous).
-            bu = torch.empty(q_c, d, rd, dtype=dtype, device=dev)
-            bv, bo_t = torch.empty_like(bu), torch.empty_like(bu)
-            bu_t = torch.empty(q_c, rd, d, dtype=dtype, device=dev)
-            bv_t, bo = torch.empty_like(bu_t), torch.empty_like(bu_t)
-            _native.check(lib.ow_fold_weights(*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype],
-                                              nw.data_ptr() if nw is not None else None, gm.data_ptr(), ch.data_ptr(),
-                                              plan.channels, q_c, d, rd, code, bu.data_ptr(), bu_t.data_ptr(),
-                                              bv.data_ptr(), bv_t.data_ptr(), bo.data_ptr(), bo_t.data_ptr(), stream),
-                          "ow_fold_weights")
-            au_t, av_t, ao_t = (a.t().contiguous() for a in (au, av, ao))
-            # Token side: P_u = A_u X', P_v = A_v X', dW' = A_o^T dY (per 16-slot tile).
-            pu = _tile_mix(lib, xt, au, None, None, d, code, stream)
-            pv = _tile_mix(lib, xt, av, None, None, d, code, stream)
-            dw = _tile_mix(lib, dyt, ao_t, None, None, d, code, stream)
-            # Channel side: batched GEMMs + the gate kernel.
-            u = torch.bmm(pu, bu)
-            v = torch.bmm(pv, bv)
-            dz = torch.bmm(dw, bo_t)
-            z, du, dv = torch.empty_like(u), torch.empty_like(u), torch.empty_like(u)
-            _native.check(lib.ow_bwd_gate(u.data_ptr(), v.data_ptr(), dz.data_ptr(), z.data_ptr(), du.data_ptr(),
-                                          dv.data_ptr(), u.numel(), code, stream), "ow_bwd_gate")
-            del u, v, dz
-            wp = torch.bmm(z, bo)
-            dpu = torch.bmm(du, bu_t)
-            dpv = torch.bmm(dv, bv_t)
-            d_bu = _slot_reduce(pu, du)   # [q_c, d, rd]
-            d_bv = _slot_reduce(pv, dv)
-            d_bo = _slot_reduce(z, dw)    # [q_c, rd, d]
-            del z, du, dv, pu, pv, dw
+        # Token-matrix gradients and dX'.
+        g_au = _tile_outer(lib, dpu, xt, d, code, stream)
+        g_av = _tile_outer(lib, dpv, xt, d, code, stream)
+        g_ao = _tile_outer(lib, dyt, wp, d, code, stream)
+        dxt = _tile_mix(lib, dpu, au_t, dpv, av_t, d, code, stream)
+        del dpu, dpv, wp, xt, dyt
 
-            # Token-matrix gradients and dX'.
-            g_au = _tile_outer(lib, dpu, xt, d, code, stream)
-            g_av = _tile_outer(lib, dpv, xt, d, code, stream)
-            g_ao = _tile_outer(lib, dyt, wp, d, code, stream)
-            dxt = _tile_mix(lib, dpu, au_t, dpv, av_t, d, code, stream)
-            del dpu, dpv, wp, xt, dyt
-
-        # dX' back to NHWC (unless a kernel wrote g), then through the RMSNorm (+ the residual's
-        # identity).
-        if not routed:
-            _native.check(lib.ow_bwd_scatter(dxt.data_ptr(), tok.data_ptr(), ch.data_ptr(),
-                                             ctypes.byref(oplan), batch, code, g.data_ptr(), stream),
-                          "ow_bwd_scatter")
-            del dxt
+        # dX' back to NHWC, then through the RMSNorm (+ the residual's identity).
+        _native.check(lib.ow_bwd_scatter(dxt.data_ptr(), tok.data_ptr(), ch.data_ptr(),
+                                         ctypes.byref(oplan), batch, code, g.data_ptr(), stream), "ow_bwd_scatter")
+        del dxt
         dx = torch.empty_like(x)
         _native.check(lib.ow_bwd_rmsnorm(x.data_ptr(), g.data_ptr(), rscale.data_ptr() if rscale is not None
                                          else None, grad.data_ptr(), dx.data_ptr(), n_rows, plan.channels,
@@ -461,10 +383,8 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
                                         g_bu.data_ptr(), g_bv.data_ptr(), g_bo.data_ptr(), g_gamma.data_ptr(),
                                         g_nw.data_ptr() if g_nw is not None else None, stream), "ow_bwd_params")
 
-    # The token-matrix gradients of the batched-GEMM path are separate tensors: into g_all too.
-    if not all(t.untyped_storage().data_ptr() == g_all.untyped_storage().data_ptr() for t in (g_au, g_av, g_ao)):
-        g_a.copy_(torch.stack([g_au.reshape(256), g_av.reshape(256), g_ao.reshape(256)]))
-    return dx, g_all
+    g_a.copy_(torch.stack([g_au.reshape(256), g_av.reshape(256), g_ao.reshape(256)]))
+    return dx, g_all, None
 
 
 def _cast_group(ts: tuple[Tensor, ...], dtypes: tuple[torch.dtype, ...]) -> tuple[Tensor, ...]:

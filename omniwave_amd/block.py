@@ -15,8 +15,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from omniwave_amd.bigemm import bigemm
-from omniwave_amd.hip import (bigemm_block_chain_hip, bigemm_block_hip, bigemm_block_s2d_hip, drop_path_scale,
-                              hip_is_supported)
+from omniwave_amd.hip import _block, _chain, bigemm_block_s2d_hip, drop_path_scale, hip_is_supported
 from omniwave_amd.routing import RoutePlan, build_route_plan
 
 RMS_EPS = 1e-6  # omniweave/models/block.py:84
@@ -114,8 +113,7 @@ class OmniWeaveBlock(nn.Module):
         if factor and (x.shape[1] % factor or x.shape[2] % factor):
             return None
         params = (self.a_u, self.a_v, self.a_o, self.b_u, self.b_v, self.b_o, self.gamma)
-        return bigemm_block_chain_hip(x, stats, self.norm_weight, self.plan, *params, factor=factor, eps=RMS_EPS,
-                                      fp8=self.fp8)
+        return _chain(x, stats, self.norm_weight, self.plan, *params, factor, RMS_EPS, self.fp8)
 
     def forward(self, x: Tensor) -> Tensor:
         """``x``: ``[B, H, W, C]`` -> ``[B, H, W, C]``."""
@@ -127,12 +125,12 @@ class OmniWeaveBlock(nn.Module):
                 raise RuntimeError("the fp8 BiGEMM variant is inference-only; call model.eval()")
             if not fused:
                 raise RuntimeError("the fp8 BiGEMM variant needs the hip backend on a gfx950 GPU")
-            return bigemm_block_hip(x, self.norm_weight, self.plan, *params, eps=RMS_EPS, fp8=True)
+            return _block(x, self.norm_weight, self.plan, *params, RMS_EPS, fp8=True)
         if fused:
             # Drop-path (block.py:99-107) fused: the kernel scales each image's rounded delta
             # before the residual; the keep mask is drawn as the reference draws it.
             scale = drop_path_scale(x.shape[0], self.drop_path_rate, x.dtype, x.device) if dropping else None
-            return bigemm_block_hip(x, self.norm_weight, self.plan, *params, eps=RMS_EPS, drop_scale=scale)
+            return _block(x, self.norm_weight, self.plan, *params, RMS_EPS, drop_scale=scale)
         variance = x.float().square().mean(dim=-1, keepdim=True)
         normalized = x * torch.rsqrt(variance.to(x.dtype) + RMS_EPS)
         normalized = (normalized * self.norm_weight).to(x.dtype)

@@ -78,22 +78,19 @@ def hip_is_supported(x: Tensor, plan: RoutePlan, b_u: Tensor) -> tuple[bool, str
 
 
 class _PackEntry:
-    __slots__ = ("refs", "versions", "packed")
+    __slots__ = ("refs", "state", "packed")
 
 
 _PACK_CACHE: OrderedDict[tuple, _PackEntry] = OrderedDict()
 _PACK_CACHE_SIZE = 64
 
 
-def _version(t: Tensor) -> int | None:
-    try:
-        return int(t._version)
-    except RuntimeError:  # inference tensors carry no version counter
-        return None
+def _state(t: Tensor) -> tuple:
+    return t.data_ptr(), t._version, t.dtype, t.shape
 
 
 def _stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def pack_weights(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_weight: Tensor | None = None,
@@ -154,32 +151,30 @@ def _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype: torch.dtype, norm_weight:
     return packed
 
 
-def _x3_supported(plan) -> bool:
-    """Whether fp32 activations of ``plan`` take the matrix-core kernel (``OW_WEIGHTS_X3``): all but
-    images of half a GiB."""
-    return bool(_native.lib().ow_weights_x3_supported(ctypes.byref(native_plan(plan))))
-
-
-def _cached_operands(norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, plan: RoutePlan,
-                     fp8: bool = False):
-    srcs = (a_u, a_v, a_o, b_u, b_v, b_o, gamma) + ((norm_weight,) if norm_weight is not None else ())
-    versions = tuple(_version(t) for t in srcs)
-    key = tuple((t.data_ptr(), t.dtype, tuple(t.shape)) for t in srcs) + (compute_dtype, plan_key(plan), fp8)
+def _cached_operands(geo: "_Geometry", norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype,
+                     layout: str) -> Tensor:
+    """The packed weights, from the cache while every parameter is the same object with the same
+    storage, shape and version (inference tensors carry no version: packed on each call)."""
+    srcs = (a_u, a_v, a_o, b_u, b_v, b_o, gamma) if norm_weight is None else (a_u, a_v, a_o, b_u, b_v, b_o, gamma,
+                                                                              norm_weight)
+    try:
+        state = [_state(t) for t in srcs]
+    except RuntimeError:
+        state = None
+    key = (compute_dtype, layout, geo.key, *map(id, srcs))
     entry = _PACK_CACHE.get(key)
-    if (entry is not None and None not in versions and entry.versions == versions
-            and all(r() is t for r, t in zip(entry.refs, srcs))):
+    if (entry is not None and state is not None and entry.state == state
+            and all([r() is t for r, t in zip(entry.refs, srcs)])):
         _PACK_CACHE.move_to_end(key)
         return entry.packed
-    entry = _PackEntry()
-    entry.refs = tuple(weakref.ref(t) for t in srcs)
-    entry.versions = versions
-    layout = "fp8" if fp8 else "x3" if compute_dtype == torch.float32 and _x3_supported(plan) else ""
-    entry.packed = _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, norm_weight, plan, gamma, layout)
-    if None not in versions:
+    packed = _pack(a_u, a_v, a_o, b_u, b_v, b_o, compute_dtype, norm_weight, geo.plan, gamma, layout)
+    if state is not None:
+        entry = _PackEntry()
+        entry.refs, entry.state, entry.packed = tuple(weakref.ref(t) for t in srcs), state, packed
         _PACK_CACHE[key] = entry
         while len(_PACK_CACHE) > _PACK_CACHE_SIZE:
             _PACK_CACHE.popitem(last=False)
-    return entry.packed
+    return packed
 
 
 def clear_pack_cache() -> None:
@@ -187,7 +182,36 @@ def clear_pack_cache() -> None:
 
 
 # ---------------------------------------------------------------------------------------
-# Custom op
+# Launch
+
+
+class _Geometry:
+    """What the calls need of a plan, derived once per set of build_route_plan's arguments."""
+
+    __slots__ = ("key", "plan", "n_tok", "native", "ref", "x3", "tables")
+
+    def __init__(self, key: tuple) -> None:
+        h, w, c, g, d, route, level = key
+        if route not in _native.OW_ROUTE:
+            raise ValueError(f"unknown route type: {route!r}")
+        self.key = key
+        self.plan = build_route_plan(h, w, c, g, d, route, level)
+        self.n_tok = h * w
+        self.native = native_plan(self.plan)
+        self.ref = ctypes.byref(self.native)  # the library only reads it
+        # fp32 activations take the matrix-core kernel (OW_WEIGHTS_X3) unless images are half a GiB
+        self.x3 = bool(_native.lib().ow_weights_x3_supported(self.ref))
+        self.tables = {}  # device -> its (token, channel) tables
+
+
+@functools.lru_cache(maxsize=256)
+def _geometry(key: tuple) -> _Geometry:
+    return _Geometry(key)
+
+
+def _key_of(desc: list[int]) -> tuple:
+    h, w, c, g, d, route, level = desc
+    return h, w, c, g, d, _ROUTE_NAME[route], level
 
 
 def _plan_desc(plan) -> list[int]:
@@ -200,8 +224,120 @@ def _plan_desc(plan) -> list[int]:
 
 
 def _plan_from_desc(desc: list[int]) -> RoutePlan:
-    h, w, c, g, d, route, level = desc
-    return build_route_plan(h, w, c, g, d, _ROUTE_NAME[route], level)
+    return _geometry(_key_of(desc)).plan
+
+
+def _tables(geo: _Geometry, device: torch.device) -> tuple[int, int]:
+    hit = geo.tables.get(device)
+    if hit is None:
+        hit = geo.tables[device] = device_tables(geo.plan, device)
+    return hit[0].data_ptr(), hit[1].data_ptr()
+
+
+def _run_forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, geo: _Geometry, flags: int, eps: float, drop_scale,
+                 want_scales: bool) -> tuple[Tensor, Tensor | None]:
+    """``bigemm_fwd`` on plain tensors: (out, row scales or None)."""
+    if not x.is_contiguous():
+        x = x.contiguous()
+    dtype, device = x.dtype, x.device
+    fuse_norm = flags & _native.OW_FUSE_NORM
+    if fuse_norm:
+        if norm_weight is None:
+            raise ValueError("OW_FUSE_NORM needs norm_weight")
+    else:
+        norm_weight = None
+    layout = ""
+    if flags & _native.OW_FUSE_FP8:
+        layout = "fp8"
+    elif dtype == torch.float32 and geo.x3:
+        layout, flags = "x3", flags | _native.OW_WEIGHTS_X3
+    packed = _cached_operands(geo, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, dtype, layout)
+    tok, ch = _tables(geo, device)
+    out = torch.empty_like(x)
+    lib = _native.lib()
+    batch = x.shape[0]
+    ws_bytes = 4 * batch * geo.n_tok if fuse_norm else 0  # ow_fwd_workspace_bytes
+    scales = torch.empty(batch * geo.n_tok, dtype=torch.float32, device=device) if want_scales and fuse_norm else None
+    # The row scales the caller asked for are the launch's scratch too.
+    workspace = scales if scales is not None else torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=device)
+    scale = _drop_scale_arg(drop_scale, x) if drop_scale is not None else None
+    if device.index != torch.cuda.current_device():
+        with torch.cuda.device(device):
+            _launch_forward(lib, x, out, eps, packed, tok, ch, geo, b_u, flags, scale, scales, workspace, ws_bytes)
+    else:
+        _launch_forward(lib, x, out, eps, packed, tok, ch, geo, b_u, flags, scale, scales, workspace, ws_bytes)
+    return out, scales
+
+
+def _launch_forward(lib, x, out, eps, packed, tok, ch, geo, b_u, flags, scale, scales, workspace, ws_bytes) -> None:
+    code, batch = _DTYPE_CODE[x.dtype], x.shape[0]
+    common = (x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(), tok, ch, geo.ref, batch,
+              b_u.shape[2], code, flags)
+    stream = _stream_ptr(x.device)
+    if scales is not None and batch:
+        written = ctypes.c_int32(0)
+        _native.check(lib.ow_bigemm_fwd_scales(*common, scale.data_ptr() if scale is not None else None,
+                                               scales.data_ptr(), ctypes.byref(written), workspace.data_ptr(), ws_bytes,
+                                               stream), "ow_bigemm_fwd_scales")
+        if not written.value:
+            _native.check(lib.ow_rms_scale(x.data_ptr(), scales.data_ptr(), scales.numel(), geo.plan.channels, eps, code,
+                                           stream), "ow_rms_scale")
+    elif scale is None:
+        _native.check(lib.ow_bigemm_fwd(*common, workspace.data_ptr(), ws_bytes, stream), "ow_bigemm_fwd")
+    else:
+        _native.check(lib.ow_bigemm_fwd_drop(*common, scale.data_ptr(), workspace.data_ptr(), ws_bytes, stream),
+                      "ow_bigemm_fwd_drop")
+
+
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
+def _plain(*tensors: Tensor | None) -> bool:
+    """Whether a call may skip the torch.library dispatcher, which costs more than a small launch:
+    plain tensors with nothing around the call that has to see the operator (compilation, tracing,
+    torch function or dispatch modes, functorch transforms such as vmap, forward-mode gradients)."""
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    for t in tensors:
+        if t is not None and type(t) not in _PLAIN:
+            return False
+    return True
+
+
+class _PlainForward(torch.autograd.Function):
+    """``bigemm_fwd`` with its gradient, for calls that ``_plain`` admits: the autograd of the custom
+    op without its dispatch."""
+
+    @staticmethod
+    def forward(ctx, x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, geo, flags, eps, drop_scale, want_scales):
+        out, scales = _run_forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, geo, flags, eps, drop_scale,
+                                   want_scales)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, drop_scale, scales)
+        ctx.plan, ctx.flags, ctx.eps = geo.plan, flags, eps
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _gradients(ctx, grad, ctx.plan)
+
+
+def _forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, flags: int, eps: float, drop_scale,
+             want_scales: bool) -> Tensor:
+    """The output of ``bigemm_fwd``, without the dispatcher where ``_plain`` allows."""
+    tensors = (x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)
+    if not _plain(*tensors, drop_scale):
+        return bigemm_fwd(*tensors, _plan_desc(plan), flags, eps, drop_scale, want_scales)[0]
+    geo = _geometry(plan_key(plan))
+    if torch.is_grad_enabled() and any([t is not None and t.requires_grad for t in tensors]):
+        return _PlainForward.apply(*tensors, geo, flags, eps, drop_scale, want_scales)
+    return _run_forward(*tensors, geo, flags, eps, drop_scale, want_scales)[0]
+
+
+# ---------------------------------------------------------------------------------------
+# Custom op
 
 
 @torch.library.custom_op("omniwave_amd::bigemm_fwd", mutates_args=())
@@ -227,44 +363,9 @@ def bigemm_fwd(
     ``want_scales`` and the RMSNorm fused, row_scale is [B * H * W] fp32, the RMSNorm scale of
     every row of x, which the backward needs (``ow_bigemm_fwd_scales``: the forward's own values
     where its kernel forms them in one place, else ``ow_rms_scale``); otherwise it is empty."""
-    plan = _plan_from_desc(plan_desc)
-    x = x.contiguous()
-    fuse_norm = bool(flags & _native.OW_FUSE_NORM)
-    if fuse_norm and norm_weight is None:
-        raise ValueError("OW_FUSE_NORM needs norm_weight")
-    fp8 = bool(flags & _native.OW_FUSE_FP8)
-    packed = _cached_operands(norm_weight if fuse_norm else None, gamma, a_u, a_v, a_o, b_u, b_v, b_o, x.dtype, plan,
-                              fp8)
-    tok, ch = device_tables(plan, x.device)
-    out = torch.empty_like(x, memory_format=torch.contiguous_format)
-    oplan = native_plan(plan)
-    lib = _native.lib()
-    ws_bytes = lib.ow_fwd_workspace_bytes(ctypes.byref(oplan), x.shape[0], flags)
-    workspace = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=x.device)
-    if x.dtype == torch.float32 and _x3_supported(plan):
-        flags |= _native.OW_WEIGHTS_X3  # the layout _cached_operands packs for fp32
-    common = (x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(), tok.data_ptr(), ch.data_ptr(),
-              ctypes.byref(oplan), x.shape[0], b_u.shape[2], _DTYPE_CODE[x.dtype], flags)
-    n_rows = x.shape[0] * plan.height * plan.width
-    scales = torch.empty(n_rows if (want_scales and fuse_norm) else 0, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        if scales.numel():
-            written = ctypes.c_int32(0)
-            scale = _drop_scale_arg(drop_scale, x) if drop_scale is not None else None
-            _native.check(lib.ow_bigemm_fwd_scales(*common, scale.data_ptr() if scale is not None else None,
-                                                   scales.data_ptr(), ctypes.byref(written), workspace.data_ptr(),
-                                                   ws_bytes, _stream_ptr(x.device)), "ow_bigemm_fwd_scales")
-            if not written.value:
-                _native.check(lib.ow_rms_scale(x.data_ptr(), scales.data_ptr(), n_rows, plan.channels, eps,
-                                               _DTYPE_CODE[x.dtype], _stream_ptr(x.device)), "ow_rms_scale")
-        elif drop_scale is None:
-            _native.check(lib.ow_bigemm_fwd(*common, workspace.data_ptr(), ws_bytes, _stream_ptr(x.device)),
-                          "ow_bigemm_fwd")
-        else:
-            scale = _drop_scale_arg(drop_scale, x)
-            _native.check(lib.ow_bigemm_fwd_drop(*common, scale.data_ptr(), workspace.data_ptr(), ws_bytes,
-                                                 _stream_ptr(x.device)), "ow_bigemm_fwd_drop")
-    return out, scales
+    out, scales = _run_forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _geometry(_key_of(plan_desc)), flags,
+                               eps, drop_scale, want_scales)
+    return out, scales if scales is not None else x.new_empty(0, dtype=torch.float32)
 
 
 def _drop_scale_arg(drop_scale: Tensor, x: Tensor) -> Tensor:
@@ -293,6 +394,11 @@ def _bigemm_fwd_setup_context(ctx, inputs, output):
 
 
 def _bigemm_fwd_backward(ctx, grad, grad_scales):
+    return _gradients(ctx, grad, _plan_from_desc(ctx.plan_desc))
+
+
+def _gradients(ctx, grad, plan):
+    """The input gradients of ``bigemm_fwd`` (five arguments after the tensors carry none)."""
     from omniwave_amd.backward import bigemm_backward
 
     if ctx.flags & _native.OW_FUSE_FP8:
@@ -300,9 +406,8 @@ def _bigemm_fwd_backward(ctx, grad, grad_scales):
     if grad is None:
         return (None,) * 14
     x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, drop_scale, scales = ctx.saved_tensors
-    grads = bigemm_backward(grad, x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o,
-                            _plan_from_desc(ctx.plan_desc), ctx.flags, ctx.eps, drop_scale=drop_scale,
-                            row_scale=scales if scales.numel() else None)
+    grads = bigemm_backward(grad, x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, ctx.flags, ctx.eps,
+                            drop_scale=drop_scale, row_scale=scales if scales is not None and scales.numel() else None)
     grads = tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad))
     return grads + (None, None, None, None, None)
 
@@ -319,7 +424,7 @@ def _require(x, plan, b_u) -> None:
 def bigemm_delta_hip(*, x, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma) -> Tensor:
     """delta for pre-normalised x (omniweave/ops/reference.py:120-173 semantics)."""
     _require(x, plan, b_u)
-    return bigemm_fwd(x, None, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _plan_desc(plan), 0, 0.0, None, False)[0]
+    return _forward(x, None, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, 0, 0.0, None, False)
 
 
 def bigemm_block_hip(x, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, eps: float = 1e-6,
@@ -332,14 +437,19 @@ def bigemm_block_hip(x, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, 
     the channel-side products on e4m3fn MFMAs (inference only; bf16 / fp16 activations).
     """
     _require(x, plan, b_u)
+    return _block(x, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, eps, residual, fp8, drop_scale)
+
+
+def _block(x, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, eps: float, residual: bool = True,
+           fp8: bool = False, drop_scale: Tensor | None = None) -> Tensor:
+    """``bigemm_block_hip`` for inputs that ``hip_is_supported`` has admitted."""
     if fp8 and x.dtype not in (torch.bfloat16, torch.float16):
         raise RuntimeError(f"hip backend not supported: the fp8 variant takes bf16 or fp16 activations, not {x.dtype}")
     flags = _native.OW_FUSE_NORM | (_native.OW_FUSE_RESIDUAL if residual else 0) | (_native.OW_FUSE_FP8 if fp8 else 0)
     # The RMSNorm row scales are kept for the backward when one will run.
     want_scales = (not fp8 and torch.is_grad_enabled()
-                   and any(t.requires_grad for t in (x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)))
-    return bigemm_fwd(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _plan_desc(plan), flags, float(eps),
-                      drop_scale, want_scales)[0]
+                   and any([t.requires_grad for t in (x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)]))
+    return _forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, flags, float(eps), drop_scale, want_scales)
 
 
 def drop_path_scale(batch: int, drop_path_rate: float, dtype: torch.dtype, device) -> Tensor:
@@ -380,30 +490,8 @@ def bigemm_fwd_s2d(
     """``space_to_depth(x + delta, factor)`` ([B, H/f, W/f, C f^2]) with the block's RMSNorm
     fused: ``ow_bigemm_fwd_rows`` with the ``ow_route_s2d_rows`` table, one pass over HBM.
     Inference only (no autograd)."""
-    plan = _plan_from_desc(plan_desc)
-    x = x.contiguous()
-    b, h, w, c = x.shape
-    if h % factor or w % factor:
-        raise ValueError(f"height {h} and width {w} must be divisible by factor {factor}")
-    fp8 = bool(flags & _native.OW_FUSE_FP8)
-    packed = _cached_operands(norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, x.dtype, plan, fp8)
-    tok, ch = device_tables(plan, x.device)
-    rows = s2d_rows_table(plan, factor, x.device)
-    out = torch.empty((b, h // factor, w // factor, c * factor * factor), dtype=x.dtype, device=x.device)
-    oplan = native_plan(plan)
-    lib = _native.lib()
-    ws_bytes = lib.ow_fwd_workspace_bytes(ctypes.byref(oplan), b, flags)
-    workspace = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        _native.check(
-            lib.ow_bigemm_fwd_rows(
-                x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(),
-                tok.data_ptr(), ch.data_ptr(), rows.data_ptr(), ctypes.byref(oplan), b, b_u.shape[2],
-                _DTYPE_CODE[x.dtype], flags, workspace.data_ptr(), ws_bytes, _stream_ptr(x.device),
-            ),
-            "ow_bigemm_fwd_rows",
-        )
-    return out
+    return _run_chain(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _geometry(_key_of(plan_desc)), flags, eps, None,
+                      factor, False)[0]
 
 
 @bigemm_fwd_s2d.register_fake
@@ -448,23 +536,35 @@ def bigemm_fwd_chain(
     [0, Q_c] with factor > 0): per output row and channel group, the sum of squares of the
     stored values, valid when ``written`` (a CPU int32 [1]) is 1; ``stats_in``: the previous
     block's ``stats`` (its RMSNorm statistics, so the launch reads only its groups' columns)."""
-    plan = _plan_from_desc(plan_desc)
+    out, stats, written = _run_chain(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _geometry(_key_of(plan_desc)),
+                                     flags, eps, stats_in, factor, True)
+    return out, stats, torch.tensor([int(written)], dtype=torch.int32)
+
+
+def _run_chain(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, geo: _Geometry, flags: int, eps: float, stats_in,
+               factor: int, want_stats: bool) -> tuple[Tensor, Tensor | None, bool]:
+    """``bigemm_fwd_chain`` (``want_stats``) or ``bigemm_fwd_s2d`` on plain tensors: (out, stats,
+    whether the launch wrote them)."""
     x = x.contiguous()
     b, h, w, c = x.shape
-    fp8 = bool(flags & _native.OW_FUSE_FP8)
-    packed = _cached_operands(norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, x.dtype, plan, fp8)
-    tok, ch = device_tables(plan, x.device)
-    q_c = ch.numel() // plan_tiles(plan)[1]
+    device = x.device
+    packed = _cached_operands(geo, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, x.dtype,
+                              "fp8" if flags & _native.OW_FUSE_FP8 else "")
+    tok, ch = _tables(geo, device)
+    q_c = geo.plan.channel_indices.shape[0]
+    stats = None
     if factor > 0:
         if h % factor or w % factor:
             raise ValueError(f"height {h} and width {w} must be divisible by factor {factor}")
-        rows = s2d_rows_table(plan, factor, x.device).data_ptr()
-        out = torch.empty((b, h // factor, w // factor, c * factor * factor), dtype=x.dtype, device=x.device)
-        stats = torch.empty((0, q_c), dtype=torch.float32, device=x.device)
+        rows = s2d_rows_table(geo.plan, factor, device).data_ptr()
+        out = torch.empty((b, h // factor, w // factor, c * factor * factor), dtype=x.dtype, device=device)
+        if want_stats:
+            stats = torch.empty((0, q_c), dtype=torch.float32, device=device)
     else:
         rows = None
         out = torch.empty_like(x)
-        stats = torch.empty((b * h * w, q_c), dtype=torch.float32, device=x.device)
+        if want_stats:
+            stats = torch.empty((b * h * w, q_c), dtype=torch.float32, device=device)
     parts = 0
     if stats_in is not None:
         if stats_in.dtype != torch.float32 or stats_in.dim() != 2 or stats_in.shape[0] != b * h * w:
@@ -472,23 +572,24 @@ def bigemm_fwd_chain(
                              f"{tuple(stats_in.shape)}")
         stats_in = stats_in.contiguous()
         parts = stats_in.shape[1]
-    oplan = native_plan(plan)
     lib = _native.lib()
-    ws_bytes = lib.ow_fwd_workspace_bytes(ctypes.byref(oplan), b, flags)
-    workspace = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=x.device)
+    ws_bytes = 4 * b * geo.n_tok  # ow_fwd_workspace_bytes (the norm is always fused here)
+    workspace = torch.empty(max(ws_bytes // 4, 1), dtype=torch.float32, device=device)
     written = ctypes.c_int32(0)
-    with torch.cuda.device(x.device):
-        _native.check(
-            lib.ow_bigemm_fwd_chain(
-                x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(),
-                tok.data_ptr(), ch.data_ptr(), rows, ctypes.byref(oplan), b, b_u.shape[2],
-                _DTYPE_CODE[x.dtype], flags, None if stats_in is None else stats_in.data_ptr(), parts,
-                stats.data_ptr() if stats.numel() else None, ctypes.byref(written),
-                workspace.data_ptr(), ws_bytes, _stream_ptr(x.device),
-            ),
-            "ow_bigemm_fwd_chain",
-        )
-    return out, stats, torch.tensor([written.value], dtype=torch.int32)
+    common = (x.data_ptr(), out.data_ptr(), eps, packed.data_ptr(), packed.numel(), tok, ch, rows, geo.ref, b,
+              b_u.shape[2], _DTYPE_CODE[x.dtype], flags)
+    with torch.cuda.device(device):
+        if want_stats:
+            _native.check(
+                lib.ow_bigemm_fwd_chain(*common, None if stats_in is None else stats_in.data_ptr(), parts,
+                                        stats.data_ptr() if stats.numel() else None, ctypes.byref(written),
+                                        workspace.data_ptr(), ws_bytes, _stream_ptr(device)),
+                "ow_bigemm_fwd_chain",
+            )
+        else:
+            _native.check(lib.ow_bigemm_fwd_rows(*common, workspace.data_ptr(), ws_bytes, _stream_ptr(device)),
+                          "ow_bigemm_fwd_rows")
+    return out, stats, bool(written.value)
 
 
 @bigemm_fwd_chain.register_fake
@@ -513,14 +614,24 @@ def bigemm_block_chain_hip(x, stats_in, norm_weight, plan, a_u, a_v, a_o, b_u, b
     launch wrote none.  The output equals the unchained call's up to the summation order of the
     RMSNorm mean of squares.  bf16 / fp16 activations, inference only."""
     _require(x, plan, b_u)
+    return _chain(x, stats_in, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, factor, eps, fp8)
+
+
+def _chain(x, stats_in, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, factor: int, eps: float,
+           fp8: bool) -> tuple[Tensor, Tensor | None]:
+    """``bigemm_block_chain_hip`` for inputs that ``hip_is_supported`` has admitted."""
     if x.dtype not in (torch.bfloat16, torch.float16):
         raise RuntimeError(f"hip backend not supported: chained blocks take bf16 or fp16, not {x.dtype}")
     if torch.is_grad_enabled() and any(t.requires_grad for t in (x, norm_weight, gamma, a_u, b_u)):
         raise RuntimeError("bigemm_block_chain_hip is inference-only (no backward); run it under torch.no_grad()")
     flags = _native.OW_FUSE_NORM | _native.OW_FUSE_RESIDUAL | (_native.OW_FUSE_FP8 if fp8 else 0)
-    out, stats, written = bigemm_fwd_chain(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, _plan_desc(plan),
-                                           flags, float(eps), stats_in, int(factor))
-    return out, (stats if int(written[0]) else None)
+    tensors = (x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)
+    if _plain(*tensors, stats_in):
+        out, stats, wrote = _run_chain(*tensors, _geometry(plan_key(plan)), flags, float(eps), stats_in, int(factor), True)
+    else:
+        out, stats, written = bigemm_fwd_chain(*tensors, _plan_desc(plan), flags, float(eps), stats_in, int(factor))
+        wrote = bool(int(written[0]))
+    return out, (stats if wrote else None)
 
 
 STEM_CHANNELS = (32, 64, 96, 128, 192, 256)

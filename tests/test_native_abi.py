@@ -273,3 +273,31 @@ def test_x3_weights_refusals_without_touching_the_gpu() -> None:
 
     assert fwd(nb, _native.OW_DTYPE_BF16) == 2 and b"OW_WEIGHTS_X3" in lib.ow_last_error()
     assert fwd(nb - 2, _native.OW_DTYPE_F32) == 1 and b"packed weights" in lib.ow_last_error()
+
+
+def test_bwd_block_refusals_without_touching_the_gpu() -> None:
+    """The single-call backward: which shapes have one, and what is refused before any launch."""
+    lib = _native.lib()
+    bf16, f32 = _native.OW_DTYPE_BF16, _native.OW_DTYPE_F32
+    flags = _native.OW_FUSE_NORM | _native.OW_FUSE_RESIDUAL
+    s3 = _native.make_plan(14, 14, 512, 16, 128, "local", 0)
+    odd = _native.make_plan(14, 14, 128, 16, 64, "local", 0)  # 13 token groups an image
+
+    def size(p, batch=2, rd=256, dtype=bf16, drop=0, scales=1):
+        return lib.ow_bwd_block_workspace(ctypes.byref(p), batch, rd, dtype, flags, drop, scales)
+
+    assert size(s3) > 0 and size(s3, dtype=f32) == 0 and size(s3, batch=-1) == 0 and size(s3, rd=192) == 0
+    assert size(odd, batch=2, rd=128) > 0 and size(odd, batch=1, rd=128) == 0
+    assert size(s3, drop=1) >= size(s3) + 2 * 196 * 512 * 2 and size(s3, scales=0) >= size(s3) + 2 * 196 * 4
+    P = ctypes.c_void_p(256)
+    small, dts = (ctypes.c_void_p * 5)(256, 256, 256, 256, 256), (ctypes.c_int32 * 5)(*[bf16] * 5)
+
+    def run(p=s3, batch=2, grads=P, ws=P, ws_bytes=size(s3), cast=None, cast_dtype=0):
+        return lib.ow_bwd_block(P, P, small, dts, P, P, P, bf16, P, None, P, P, ctypes.byref(p), batch, 256, bf16, flags,
+                                1e-6, P, grads, cast, cast_dtype, ws, ws_bytes, None)
+
+    assert run(p=odd, batch=1) == 2 and b"single-call" in lib.ow_last_error()
+    assert run(grads=None) == 1 and b"NULL" in lib.ow_last_error()
+    assert run(ws_bytes=size(s3) - 1) == 1 and b"workspace" in lib.ow_last_error()
+    assert run(ws=ctypes.c_void_p(264)) == 1 and b"workspace" in lib.ow_last_error()
+    assert run(cast=P, cast_dtype=f32) == 1 and b"cast" in lib.ow_last_error()
