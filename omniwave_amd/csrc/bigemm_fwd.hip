@@ -113,19 +113,57 @@ __global__ void __launch_bounds__(kThreads) rms_rows16_kernel(RmsArgs a) {
   }
 }
 
-// Any C: one wave per row, element loads.
-template <class Ty>
-__global__ void __launch_bounds__(kThreads) rms_rows_generic_kernel(RmsArgs a) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
-  if (row >= a.rows) return;
-  float acc = 0.0f;
-  for (int c = lane; c < a.channels; c += 64) {
-    const float v = Ty::to_f32(a.x[row * a.channels + c]);
-    acc = fmaf(v, v, acc);
+// Any C and alignment: LPR lanes per row, 8 values per lane step (16-byte loads at any address),
+// NR rows per lane group in flight.  One wave per row with 2-byte loads was bound by its own
+// instructions: 102400 rows of 96 took 15.2 us, 5.9 now.
+template <class Ty, int LPR, int NR>
+__global__ void __launch_bounds__(kThreads) rms_rows_any_kernel(RmsArgs a) {
+  constexpr int RPP = kThreads / LPR;      // rows per pass of the workgroup
+  const int sub = threadIdx.x % LPR;
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * (RPP * NR) + threadIdx.x / LPR;
+  const uint16_t* end = a.x + a.rows * a.channels;
+  float acc[NR] = {};
+  for (int c = 8 * sub; c < a.channels; c += 8 * LPR) {
+    u32x4 v[NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int64_t row = row0 + k * RPP;
+      v[k] = load_ragged8(a.x + row * a.channels + c, row < a.rows ? a.channels - c : 0, end);
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int64_t row = row0 + k * RPP;
+      v[k] = finish_ragged8(v[k], a.x + row * a.channels + c, row < a.rows ? a.channels - c : 0, end);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[k] = Ty::dot2sq(v[k][e], acc[k]);
+    }
   }
-  for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
-  if (lane == 0) a.scale[row] = rms_scale<Ty>(acc / static_cast<float>(a.channels), a.eps);
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    for (int m = LPR >> 1; m > 0; m >>= 1) acc[k] += __shfl_xor(acc[k], m);
+    const int64_t row = row0 + k * RPP;
+    if (sub == 0 && row < a.rows) a.scale[row] = rms_scale<Ty>(acc[k] / static_cast<float>(a.channels), a.eps);
+  }
+}
+
+template <class Ty>
+int launch_rms_any(const RmsArgs& a, hipStream_t s) {
+  auto launch = [&](auto lpr) {
+    constexpr int L = decltype(lpr)::value, per = kThreads / L;
+    // Four rows per lane group once that still leaves four workgroups per CU, else one.
+    const bool four = a.rows >= static_cast<int64_t>(4) * 4 * per * device_cus();
+    const dim3 g(static_cast<unsigned>((a.rows + per * (four ? 4 : 1) - 1) / (per * (four ? 4 : 1))));
+    if (four)
+      hipLaunchKernelGGL((rms_rows_any_kernel<Ty, L, 4>), g, dim3(kThreads), 0, s, a);
+    else
+      hipLaunchKernelGGL((rms_rows_any_kernel<Ty, L, 1>), g, dim3(kThreads), 0, s, a);
+    return hip_status(hipGetLastError(), "rms_rows_any_kernel launch");
+  };
+  // The narrowest power of two of lanes that takes a row in one step, up to a wave.
+  if (a.channels <= 64) return launch(std::integral_constant<int, 8>{});
+  if (a.channels <= 128) return launch(std::integral_constant<int, 16>{});
+  if (a.channels <= 256) return launch(std::integral_constant<int, 32>{});
+  return launch(std::integral_constant<int, 64>{});
 }
 
 // ---------------------------------------------------------------------------------------
@@ -166,7 +204,9 @@ struct FwdArgs {
 //   kModeStrided  group qc is columns res + k*n, k < d, n = q_c in {2, 4, 8}, C = n*d (radix
 //                 levels >= 1, omniweave/models/routing.py:107-121): every 16-byte vector of
 //                 a row holds 8/n consecutive tile columns of the group
-//   kModeElement  anything else (padded groups, unaligned or ragged rows): element access
+//   kModeRagged   contiguous groups with a partial last one, rows of any width and alignment:
+//                 16-byte vectors at any address, the last one of a row cut off
+//   kModeElement  anything else (strided ragged groups, unaligned strided rows): element access
 // (kModeContig, kModeStrided, kModeElement: ow_device.h)
 constexpr int kBatch = 16;  // global loads kept in flight per thread by the gather / scatter loops
 
@@ -372,6 +412,26 @@ bigemm_fwd_kernel(FwdArgs a) {
       const int64_t id = rowid[idx / VPR];
       v[i] = u32x4{0u, 0u, 0u, 0u};
       if (id >= 0) v[i] = *reinterpret_cast<const u32x4*>(a.x + id * a.channels + qc * D + (idx % VPR) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kThreads;
+      *reinterpret_cast<u32x4*>(&xs[(idx / VPR) * LDX + (idx % VPR) * 8]) = v[i];
+    }
+  } else if (a.mode == kModeRagged) {
+    // As kModeContig at any address: 40x40x95, B = 64 takes 40 us with its statistics pass, 69
+    // with element access and the pass of then.
+    constexpr int VPR = D / 8;
+    constexpr int NV = ROWS * VPR / kThreads;
+    const uint16_t* end = a.x + static_cast<int64_t>(a.batch) * a.n_tok * a.channels;
+    u32x4 v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kThreads;
+      const int64_t id = rowid[idx / VPR];
+      const int c = qc * D + (idx % VPR) * 8, n = id >= 0 ? a.channels - c : 0;
+      const uint16_t* p = a.x + id * a.channels + c;
+      v[i] = finish_ragged8(load_ragged8(p, n, end), p, n, end);
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -796,6 +856,32 @@ bigemm_fwd_kernel(FwdArgs a) {
     else if (a.stride == 2) store_rows(std::integral_constant<int, 4>{});
     else if (a.stride == 4) store_rows(std::integral_constant<int, 2>{});
     else store_rows(std::integral_constant<int, 1>{});
+  } else if (a.mode == kModeRagged) {
+    constexpr int VPR = D / 8, RPI = 64 / VPR, NIT = 32 / RPI;  // lanes per row, rows per pass, passes
+    const int sub = lane % VPR, rsub = lane / VPR, c = qc * D + 8 * sub;
+    const uint16_t* end = a.x + static_cast<int64_t>(a.batch) * a.n_tok * a.channels;
+    u32x4 val[NIT], xv[NIT];
+    int32_t ids[NIT];
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+      const int r = wave * 32 + rsub + RPI * k;
+      ids[k] = rowout[r];
+      const int32_t in = rowid[r];  // >= 0 wherever the output row is
+      val[k] = *reinterpret_cast<const u32x4*>(&xs[r * LDX + 8 * sub]);
+      const int n = a.residual && in >= 0 ? a.channels - c : 0;
+      const uint16_t* p = a.x + static_cast<int64_t>(in) * a.channels + c;
+      xv[k] = finish_ragged8(load_ragged8(p, n, end), p, n, end);
+    }
+    if (a.residual) {
+#pragma unroll
+      for (int k = 0; k < NIT; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) val[k][e] = add_residual2<Ty>(xv[k][e], val[k][e]);
+    }
+#pragma unroll
+    for (int k = 0; k < NIT; ++k)
+      if (ids[k] >= 0)
+        store_ragged8(a.out + static_cast<int64_t>(ids[k]) * a.channels + c, a.channels - c, val[k]);
   } else {
     constexpr int NE = ROWS * D / kThreads;
 #pragma unroll 4
@@ -1104,10 +1190,7 @@ int launch_rms(const RmsArgs& a, hipStream_t s) {
     case 64: hipLaunchKernelGGL((rms_rows_kernel<Ty, 64>), dim3(blocks8), dim3(kThreads), 0, s, a); break;
     case 128: hipLaunchKernelGGL((rms_rows_kernel<Ty, 128>), dim3(blocks8), dim3(kThreads), 0, s, a); break;
     case 256: hipLaunchKernelGGL((rms_rows_kernel<Ty, 256>), dim3(blocks8), dim3(kThreads), 0, s, a); break;
-    default: {
-      const unsigned blocks = static_cast<unsigned>((a.rows + kWaves - 1) / kWaves);
-      hipLaunchKernelGGL(rms_rows_generic_kernel<Ty>, dim3(blocks), dim3(kThreads), 0, s, a);
-    }
+    default: return launch_rms_any<Ty>(a, s);
   }
   return hip_status(hipGetLastError(), "rms_rows_kernel launch");
 }
@@ -1174,7 +1257,18 @@ FwdPath fwd_path(const void* x, const void* out, const OwPlan* plan, int32_t q_c
     p.mode = kModeContig;
   else if (vec_ok && !identity && c == q_c * d && (q_c == 2 || q_c == 4 || q_c == 8))
     p.mode = kModeStrided;
+  else if (identity)
+    p.mode = kModeRagged;
   return p;
+}
+
+// bf16 / f16 launches of the 16-token-unit kernel (16-byte aligned tensors).
+bool fwd_uses_wave16(const void* x, const void* out, const OwPlan* plan, int32_t q_c, int32_t rd, int32_t dtype,
+                     int32_t flags, int32_t batch) {
+  if ((dtype != OW_DTYPE_BF16 && dtype != OW_DTYPE_F16) || (flags & OW_FUSE_FP8)) return false;
+  const int64_t elems = static_cast<int64_t>(batch) * plan->height * plan->width * plan->channels;
+  return aligned16(x) && aligned16(out) &&
+         wave16_supported(plan->channel_tile, rd, plan->channels, q_c, plan->radix_level == 0, elems);
 }
 
 // d = 128, rd = 256 launches with contiguous channel groups and 16-byte aligned rows (bf16 /
@@ -1200,7 +1294,8 @@ bool fwd_needs_scale_buffer(const void* x, const void* out, const OwPlan* plan, 
   if (ow_plan_dims(plan, &q_s, &q_c) != OW_OK) return false;
   const FwdPath p = fwd_path(x, out, plan, q_c, dtype, flags);
   if (p.resident && rd == 2 * plan->channel_tile) return false;
-  if (p.mode == kModeElement) return true;
+  if (fwd_uses_wave16(x, out, plan, q_c, rd, dtype, flags, batch)) return false;
+  if (p.mode == kModeElement || p.mode == kModeRagged) return true;
   if (stats_in) return false;
   // The persistent kernel reads whole rows only for strided groups (and forms their scales);
   // with contiguous groups its scales come from the statistics pass (measured: cheaper than
@@ -1361,17 +1456,10 @@ int ow_rms_scale(const void* x, float* scale, int64_t rows, int32_t channels, fl
   }
   ow::RmsArgs r{static_cast<const uint16_t*>(x), scale, rows, channels, eps};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!ow::aligned16(x)) {  // element path
-    const unsigned blocks = static_cast<unsigned>((rows + ow::kWaves - 1) / ow::kWaves);
-    if (dtype == OW_DTYPE_BF16)
-      hipLaunchKernelGGL(ow::rms_rows_generic_kernel<ow::BF16>, dim3(blocks), dim3(ow::kThreads), 0, s, r);
-    else
-      hipLaunchKernelGGL(ow::rms_rows_generic_kernel<ow::F16>, dim3(blocks), dim3(ow::kThreads), 0, s, r);
-    if (int rc = ow::hip_status(hipGetLastError(), "rms_rows_generic_kernel launch")) return rc;
-  } else {
-    const int rc = dtype == OW_DTYPE_BF16 ? ow::launch_rms<ow::BF16>(r, s) : ow::launch_rms<ow::F16>(r, s);
-    if (rc) return rc;
-  }
+  const bool any = !ow::aligned16(x);
+  const int rc = dtype == OW_DTYPE_BF16 ? (any ? ow::launch_rms_any<ow::BF16>(r, s) : ow::launch_rms<ow::BF16>(r, s))
+                                        : (any ? ow::launch_rms_any<ow::F16>(r, s) : ow::launch_rms<ow::F16>(r, s));
+  if (rc) return rc;
   ow::clear_error();
   return OW_OK;
 }
@@ -1420,7 +1508,8 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
 
   const bool fp32 = dtype == OW_DTYPE_F32;
   const ow::FwdPath path = ow::fwd_path(x, out, plan, q_c, dtype, flags);
-  const bool resident = path.resident && rd == 2 * d;
+  const bool wave16 = ow::fwd_uses_wave16(x, out, plan, q_c, rd, dtype, flags, batch);
+  const bool resident = wave16 || (path.resident && rd == 2 * d);
   const int32_t mode = path.mode;
   float* scale = nullptr;
   // scale_out (ow_bigemm_fwd_scales): the row scales go to the caller's buffer where the launch
@@ -1473,8 +1562,6 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
     r.residual = (flags & OW_FUSE_RESIDUAL) ? 1 : 0;
     r.eps = eps;
     r.drop_scale = drop_scale;
-    const int64_t x_elems = static_cast<int64_t>(batch) * n * c;
-    const bool wave16 = ow::wave16_supported(d, rd, c, q_c, x_elems);
     if (wave16 && want_scales) {
       r.rs_out = scale_out;
       *scale_written = 1;

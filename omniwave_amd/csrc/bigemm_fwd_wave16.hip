@@ -27,6 +27,9 @@
 //   * the accumulator of each 16x16 product is, pair of accumulators by pair, the next product's
 //     operand: its rows 4h + i (h = lane / 16) are the K slots kord16(j, h) = 16 (j / 4) + 4h +
 //     j % 4 of the next 16x16x32 operand, the order the packed weights use (pack16_kernel);
+//   * a last group cut off by the row's end (contiguous groups, whole 16-byte pieces): the row
+//     stride is the tensor's own, and pieces past it go past the buffer, so they read as zero
+//     and aren't stored;
 //   * twelve waves (three per SIMD) per CU, two groups' packed weights (96 KB) in LDS, units
 //     drawn one at a time from the workgroup's range through an LDS counter.
 #include <hip/hip_runtime.h>
@@ -101,11 +104,12 @@ struct UnitEntry {
   int32_t tk, to, b;
 };
 
-template <class Ty, int QC, bool SG, bool OM, bool DROP>
+template <class Ty, int QC, bool SG, bool OM, bool DROP, bool RG = false>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads), amdgpu_waves_per_eu(3, 3)))
 bigemm_fwd_wave16_kernel(ResidentArgs a, int32_t n_units) {
   static_assert(QC == 2 || QC == 4, "two or four channel groups");
-  constexpr int kCT = QC * kD;  // channels of a row of x and out
+  static_assert(!(RG && SG), "a cut-off group needs contiguous groups");
+  const int kCT = RG ? a.channels : QC * kD;  // channels of a row of x and out
   __shared__ __attribute__((aligned(16))) Wave16Lds sh;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = lane >> 4, l16 = lane & 15;
@@ -178,14 +182,16 @@ bigemm_fwd_wave16_kernel(ResidentArgs a, int32_t n_units) {
   // Rows of the unit whose token-l16 input row is `in`: load k holds token 4k + h, piece l16
   // (q_c = 4: xr the piece of the 256-byte half at byte own_off, xo of the other half).
   const uint32_t own_off = (QC == 4 && !SG) ? 256u * ph : 0u;
+  const bool own_in = !RG || own_off + 16u * l16 < 2u * kCT, other_in = !RG || 256u - own_off + 16u * l16 < 2u * kCT;
   u32x4 xr[4], xo[QC == 4 ? 4 : 1];
   auto load_rows = [&](int32_t in) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int32_t row = __shfl(in, 4 * k + h, 16);
       const uint32_t off = row >= 0 ? static_cast<uint32_t>(row) * (kCT * 2u) + 16u * l16 : kOutOfRange;
-      xr[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, off + own_off, 0, 0);
-      if constexpr (QC == 4) xo[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, off + (256u - own_off), 0, 0);
+      xr[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, own_in ? off + own_off : kOutOfRange, 0, 0);
+      if constexpr (QC == 4)
+        xo[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, other_in ? off + (256u - own_off) : kOutOfRange, 0, 0);
     }
   };
 
@@ -427,7 +433,7 @@ bigemm_fwd_wave16_kernel(ResidentArgs a, int32_t n_units) {
         ov = *reinterpret_cast<const u32x4*>(&tile[toff(t, 8 * l16)]);
       }
       const uint32_t off =
-          orow >= 0 ? static_cast<uint32_t>(orow) * (kCT * 2u) + own_off + 16u * l16 : kOutOfRange;
+          orow >= 0 && own_in ? static_cast<uint32_t>(orow) * (kCT * 2u) + own_off + 16u * l16 : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(ov, ro, off, 0, 0);
     }
     // The next unit overwrites the tile and the tables: every lane's reads above are done.
@@ -437,7 +443,7 @@ bigemm_fwd_wave16_kernel(ResidentArgs a, int32_t n_units) {
   }
 }
 
-template <class Ty, int QC, bool SG>
+template <class Ty, int QC, bool SG, bool RG = false>
 int launch_sg(const ResidentArgs& a, hipStream_t stream) {
   const int32_t n_units = static_cast<int32_t>(static_cast<int64_t>(a.batch) * a.q_s);
   const int64_t want = (static_cast<int64_t>(n_units) + kWaves - 1) / kWaves;  // unit ranges
@@ -456,25 +462,33 @@ int launch_sg(const ResidentArgs& a, hipStream_t stream) {
   if (a.out_tok && a.drop_scale) return fail(OW_ERR_UNSUPPORTED, "an output-row table with a drop-path scale");
   const dim3 g(static_cast<unsigned>(grid)), b(kThreads);
   if (a.out_tok)
-    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, true, false>), g, b, 0, stream, a, n_units);
+    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, true, false, RG>), g, b, 0, stream, a, n_units);
   else if (a.drop_scale)
-    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, false, true>), g, b, 0, stream, a, n_units);
+    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, false, true, RG>), g, b, 0, stream, a, n_units);
   else
-    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, false, false>), g, b, 0, stream, a, n_units);
+    hipLaunchKernelGGL((bigemm_fwd_wave16_kernel<Ty, QC, SG, false, false, RG>), g, b, 0, stream, a, n_units);
   return hip_status(hipGetLastError(), "bigemm_fwd_wave16_kernel launch");
 }
 
 template <class Ty>
 int launch_ty(const ResidentArgs& a, bool interleaved, hipStream_t stream) {
+  if (a.channels != a.q_c * kD)
+    return a.q_c == 4 ? launch_sg<Ty, 4, false, true>(a, stream) : launch_sg<Ty, 2, false, true>(a, stream);
   if (a.q_c == 4) return interleaved ? launch_sg<Ty, 4, true>(a, stream) : launch_sg<Ty, 4, false>(a, stream);
   return interleaved ? launch_sg<Ty, 2, true>(a, stream) : launch_sg<Ty, 2, false>(a, stream);
 }
 
 }  // namespace
 
-bool wave16_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c, int64_t x_elems) {
+// A cut-off last group is taken while its rows are whole 16-byte pieces: the channel side then
+// works up to half its time for padding, and still beats the streamed kernel, whose weights don't
+// stay in LDS and whose scales need a pass of their own (B = 64, 40x40x96: 23.9 us against 39.9
+// at 95 channels, which the streamed kernel takes; B = 32, 40x40x200: 25.0 against 39.5 at 199).
+bool wave16_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c, bool contiguous, int64_t x_elems) {
+  const bool whole = channels == q_c * kD;
+  const bool cut = contiguous && channels % 8 == 0 && channels > (q_c - 1) * kD && channels < q_c * kD;
   // Byte offsets are 32-bit and kOutOfRange (2^31) must lie past x and out.
-  return d == kD && rd == kRD && (q_c == 2 || q_c == 4) && channels == q_c * kD && x_elems * 2 < (int64_t(1) << 31);
+  return d == kD && rd == kRD && (q_c == 2 || q_c == 4) && (whole || cut) && x_elems * 2 < (int64_t(1) << 31);
 }
 
 int launch_fwd_wave16(const ResidentArgs& a, int32_t radix_level, int32_t dtype, hipStream_t stream) {

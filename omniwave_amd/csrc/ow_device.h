@@ -21,6 +21,7 @@ namespace ow {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;  // 16 bytes at any 16-bit value's address
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -734,6 +735,40 @@ __device__ __forceinline__ void pair_output_t(const f32x16 (&W)[MB], u32x4 ao, i
   for (int mb = 0; mb < MB; ++mb) dl[mb] = Ty::mma32(pack_kstep<Ty>(W[mb], 1), ao1, dl[mb]);
 }
 
+// Values 0..7 of a row from p on, of which the first n lie in the row (the rest read as zero), at
+// any address; end: one past the tensor.  A vector that reaches past its row is read whole while
+// it stays inside the tensor (the next row's values are dropped).  Two steps, so that a caller
+// with several vectors has all their loads in flight: load_ragged8 issues the load,
+// finish_ragged8 cuts the vector off and reads the tensor's last one by elements.
+__device__ __forceinline__ u32x4 load_ragged8(const uint16_t* p, int n, const uint16_t* end) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (n > 0 && p + 8 <= end) v = *reinterpret_cast<const u32x4_any*>(p);
+  return v;
+}
+__device__ __forceinline__ u32x4 finish_ragged8(u32x4 v, const uint16_t* p, int n, const uint16_t* end) {
+  if (n > 0 && p + 8 > end) {
+    for (int j = 0; j < n; ++j) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (w == j >> 1) v[w] |= static_cast<uint32_t>(p[j]) << (16 * (j & 1));
+    }
+  }
+#pragma unroll
+  for (int w = 0; w < 4; ++w) v[w] &= n >= 2 * w + 2 ? 0xffffffffu : n == 2 * w + 1 ? 0xffffu : 0u;
+  return v;
+}
+
+// The first n of 8 values to p.
+__device__ __forceinline__ void store_ragged8(uint16_t* p, int n, const u32x4& v) {
+  if (n >= 8) {
+    *reinterpret_cast<u32x4_any*>(p) = v;
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 7; ++j)
+    if (j < n) p[j] = j & 1 ? hi16(v[j >> 1]) : lo16(v[j >> 1]);
+}
+
 inline int hip_status(hipError_t e, const char* what) {
   if (e == hipSuccess) return OW_OK;
   return fail(OW_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
@@ -781,6 +816,7 @@ bool resident_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c);
 constexpr int kModeContig = 0;
 constexpr int kModeStrided = 1;
 constexpr int kModeElement = 2;
+constexpr int kModeRagged = 3;
 struct FwdPath {
   bool resident;
   int32_t mode;
@@ -826,9 +862,9 @@ bool fwd_uses_persist(const void* x, const void* out, const OwPlan* plan, int32_
                       int32_t batch);
 
 // 16-token-unit forward for d = 64, rd = 128, C = 64 q_c with q_c in {2, 4} (contiguous groups,
-// or the interleaved groups of radix levels >= 1; bigemm_fwd_wave16.hip); reads the packed
-// weights' second section (packed16_elems).
-bool wave16_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c, int64_t x_elems);
+// the last one whole or cut off at a multiple of 8 channels, or the interleaved groups of radix
+// levels >= 1; bigemm_fwd_wave16.hip); reads the packed weights' second section (packed16_elems).
+bool wave16_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c, bool contiguous, int64_t x_elems);
 int launch_fwd_wave16(const ResidentArgs& a, int32_t radix_level, int32_t dtype, hipStream_t stream);
 
 // fp32 path (bigemm_fwd_f32.hip): operand packing, RMSNorm row scales and the forward.
