@@ -1284,8 +1284,19 @@ bool fwd_uses_persist(const void* x, const void* out, const OwPlan* plan, int32_
   return persist_supported(plan->channel_tile, rd, plan->channels, q_c, elems);
 }
 
+// Whether a launch that takes the persistent kernel is small enough for its split form.
+bool fwd_uses_split(const OwPlan* plan, int32_t q_s, int32_t q_c, int32_t flags, int32_t batch) {
+  return !(flags & OW_FUSE_FP8) && split_supported(static_cast<int64_t>(batch) * q_s, q_c);
+}
+
+// Contiguous groups whose row sums the split kernel forms itself, in the order of
+// rms_rows16_kernel (same scales).
+bool split_inline(int32_t q_c) { return q_c == 1 || q_c == 2 || q_c == 4 || q_c == 8; }
+
 // The RMSNorm row scales of a launch come from one of four places (kNorm*); only kNormBuffer
-// (and the fp32 kernel with OW_FUSE_NORM) uses the workspace, for batch * H * W floats.
+// (and the fp32 kernel with OW_FUSE_NORM) uses the workspace, for batch * H * W floats.  What a
+// caller has to provide doesn't depend on the batch or on a last group's width: small launches
+// and cut-off groups that form their scales themselves ask for the workspace all the same.
 bool fwd_needs_scale_buffer(const void* x, const void* out, const OwPlan* plan, int32_t rd, int32_t dtype,
                             int32_t flags, bool stats_in, int32_t batch) {
   if (!(flags & OW_FUSE_NORM)) return false;
@@ -1294,7 +1305,6 @@ bool fwd_needs_scale_buffer(const void* x, const void* out, const OwPlan* plan, 
   if (ow_plan_dims(plan, &q_s, &q_c) != OW_OK) return false;
   const FwdPath p = fwd_path(x, out, plan, q_c, dtype, flags);
   if (p.resident && rd == 2 * plan->channel_tile) return false;
-  if (fwd_uses_wave16(x, out, plan, q_c, rd, dtype, flags, batch)) return false;
   if (p.mode == kModeElement || p.mode == kModeRagged) return true;
   if (stats_in) return false;
   // The persistent kernel reads whole rows only for strided groups (and forms their scales);
@@ -1511,6 +1521,8 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
   const bool wave16 = ow::fwd_uses_wave16(x, out, plan, q_c, rd, dtype, flags, batch);
   const bool resident = wave16 || (path.resident && rd == 2 * d);
   const int32_t mode = path.mode;
+  const bool persist = ow::fwd_uses_persist(x, out, plan, rd, dtype, flags, batch);
+  const bool split = persist && ow::fwd_uses_split(plan, q_s, q_c, flags, batch);
   float* scale = nullptr;
   // scale_out (ow_bigemm_fwd_scales): the row scales go to the caller's buffer where the launch
   // forms them in one place (the statistics pass, or the 16-token kernel below).
@@ -1524,8 +1536,10 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
                    need);
       scale = static_cast<float*>(workspace);
     }
-    if (int rc = ow_rms_scale(x, scale, static_cast<int64_t>(batch) * n, c, eps, dtype, stream)) return rc;
-    if (want_scales) *scale_written = 1;
+    if (wave16 || (split && ow::split_inline(q_c))) {
+      scale = nullptr;  // the kernel forms the scales itself
+    } else if (int rc = ow_rms_scale(x, scale, static_cast<int64_t>(batch) * n, c, eps, dtype, stream)) return rc;
+    if (want_scales && scale) *scale_written = 1;
   }
 
   if (x3) {
@@ -1572,7 +1586,7 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
     if (rc == OW_OK) ow::clear_error();
     return rc;
   }
-  if (ow::fwd_uses_persist(x, out, plan, rd, dtype, flags, batch)) {
+  if (persist) {
     ow::PersistArgs p{};
     p.x = static_cast<const uint16_t*>(x);
     p.out = static_cast<uint16_t*>(out);
@@ -1600,14 +1614,19 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
         p.row_scale = stats_in;
         p.parts = stats_in_parts;
       } else {
-        p.norm = ow::kNormInline;  // strided groups: scales from the whole-row tile fetch
+        p.norm = ow::kNormInline;  // strided groups and small launches: scales from whole rows
+        if (split && want_scales) {
+          p.rs_out = scale_out;
+          *scale_written = 1;
+        }
       }
     }
     if (stats_out && !out_rows) {
       p.stats_out = stats_out;
       if (stats_written) *stats_written = 1;
     }
-    const int rc = ow::launch_fwd_persist(p, dtype, s);
+    const int rc = split ? ow::launch_fwd_split(p, dtype, s) : ow::launch_fwd_persist(p, dtype, s);
+    if (rc != OW_OK && scale_written) *scale_written = 0;
     if (rc == OW_OK) ow::clear_error();
     return rc;
   }

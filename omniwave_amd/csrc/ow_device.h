@@ -854,9 +854,14 @@ struct PersistArgs {
   int32_t fp8;              // V' on the e4m3 MFMA (fp8 packed weights)
   const int32_t* chan;      // [q_c * 128] channel table (strided groups: the first entry of a group)
   int32_t stride;           // 1: contiguous groups; 2, 4, 8: strided groups (= q_c)
+  float* rs_out;            // split kernel with kNormInline: NULL, or [batch * n_tok]: the rows' scales
 };
 bool persist_supported(int32_t d, int32_t rd, int32_t channels, int32_t q_c, int64_t x_elems);
 int launch_fwd_persist(const PersistArgs& a, int32_t dtype, hipStream_t stream);
+// The persistent kernel's launches (without fp8) with few token groups, the expanded dimension
+// split over the waves of a workgroup (bigemm_fwd_split.hip).
+bool split_supported(int64_t n_groups, int32_t q_c);
+int launch_fwd_split(const PersistArgs& a, int32_t dtype, hipStream_t stream);
 // Whether a bf16 / f16 launch takes the persistent kernel.
 bool fwd_uses_persist(const void* x, const void* out, const OwPlan* plan, int32_t rd, int32_t dtype, int32_t flags,
                       int32_t batch);
