@@ -456,6 +456,34 @@ int ow_bwd_param_reduce128(const void* pu, const void* pv, const void* dw, const
                            const void* dv, float* partial, int64_t n_partial, int64_t slots, int32_t q_c, int32_t rd,
                            int32_t dtype, void* stream);
 
+/* The fp32 backward's channel side on the bf16 matrix cores, every fp32 operand as three bf16
+ * parts and a product as the six part products above 2^-24 (replaces ow_tile_mix, ow_tile_outer,
+ * ow_bwd_gate, ow_bwd_scatter and the channel GEMMs; the reference's fp32 autograd recompute,
+ * omniweave/ops/triton.py:256-292).  ow_pack_bwd_x3: the folded weights (as ow_fold_weights; formed
+ * in fp64) in parts, ow_bwd_x3_packed_bytes(q_c, d, rd) bytes (0: unsupported shape).
+ * ow_bwd_channel_x3: from the fp32 tiles X', dY ([q_c][slots][d], ow_bwd_gather), P_u, P_v, dW'
+ * ([q_c][slots][d]) and Z, dU', dV' ([q_c][slots][rd]) as ow_bwd_channel, then dX' written to
+ * g [rows][channels] at its routed place (every element once) and the token-matrix gradients
+ * dA_u, dA_v, dA_o to d_a [3][256] (partial: workspace of n_partial =
+ * ow_bwd_channel_x3_partials(slots, q_c) rows of 768 floats, summed in fp64).  ow_bwd_param_reduce_x3: dB_u'', dB_v'' ([d][rd] per group) and
+ * dB_o'' ([rd][d]) as partial[ranges][3][q_c][d * rd], summed by the caller over the ranges
+ * (ow_bwd_param_reduce_x3_ranges gives a count that fits the device).  slots % 16 == 0, d in
+ * {64, 128}, rd in {128, 256}; tile buffers 16-byte aligned. */
+size_t ow_bwd_x3_packed_bytes(int32_t q_c, int32_t d, int32_t rd);
+int ow_pack_bwd_x3(const void* b_u, const void* b_v, const void* b_o, int32_t weight_dtype, const float* norm_weight,
+                   const float* gamma, const int32_t* channel_index, int32_t channels, int32_t q_c, int32_t d,
+                   int32_t rd, void* packed, size_t packed_bytes, void* stream);
+int64_t ow_bwd_channel_x3_partials(int64_t slots, int32_t q_c);
+int ow_bwd_channel_x3(const float* xt, const float* dyt, const float* a_u, const float* a_v, const float* a_o,
+                      const void* packed, size_t packed_bytes, float* pu, float* pv, float* dw, float* z, float* du,
+                      float* dv, const int32_t* token_index, const int32_t* channel_index, int64_t slots, int32_t n_tok,
+                      int32_t channels, int32_t q_s, int32_t q_c, int32_t d, int32_t rd, float* g, float* partial,
+                      int64_t n_partial, float* d_a, void* stream);
+int64_t ow_bwd_param_reduce_x3_ranges(int64_t slots, int32_t q_c);
+int ow_bwd_param_reduce_x3(const float* pu, const float* pv, const float* dw, const float* z, const float* du,
+                           const float* dv, float* partial, int64_t ranges, int64_t slots, int32_t q_c, int32_t d,
+                           int32_t rd, void* stream);
+
 /* out[c] = sum over r < rows of partial[r * cols + c], fp32, in a fixed order for given rows
  * and cols (run to run identical): the sums of the per-workgroup partials above and of the
  * token-matrix partials of ow_bwd_fused / ow_bwd_channel2 (the reference's autograd sums them

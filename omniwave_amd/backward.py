@@ -5,7 +5,7 @@ Replaces the fp32 autograd recompute of the accelerated backend
 accumulation, entirely on the HIP stream of the gradient:
 
 * for bf16 / fp16 one native call (``ow_bwd_block``) launches the kernels below in order; fp32 and
-  d = 64 with an odd number of token groups are composed here;
+  16-bit d = 64 with an odd number of token groups are composed here;
 * routing, RMSNorm, gate and parameter fold-back are the libomniwave_amd.so kernels
   (``ow_bwd_gather``, ``ow_bwd_gate``, ``ow_bwd_scatter``, ``ow_bwd_rmsnorm``,
   ``ow_bwd_params``, ``ow_fold_weights``);
@@ -16,13 +16,15 @@ accumulation, entirely on the HIP stream of the gradient:
   dX', W' and the token-matrix gradients; with the identity channel order their ``_routed``
   forms read x / dy and write dX' straight to the NHWC gradient, so neither the gather nor the
   scatter pass runs);
-  otherwise (fp32) the 16x16 token-side products are
-  ``ow_tile_mix`` / ``ow_tile_outer`` (16x16x16 MFMA) around plain batched GEMMs over all slots
-  of a channel group (``torch.bmm`` -> hipBLASLt, every right operand contiguous) and
+* for fp32 three kernels on the bf16 matrix cores (``ow_bwd_channel_x3``: two of them, and
+  ``ow_bwd_param_reduce_x3``), every operand in three bf16 parts;
+* otherwise (16 bits, d = 64 with an odd number of token groups) the 16x16 token-side products
+  are ``ow_tile_mix`` / ``ow_tile_outer`` (16x16x16 MFMA) around plain batched GEMMs over all
+  slots of a channel group (``torch.bmm`` -> hipBLASLt, every right operand contiguous) and
   ``ow_bwd_gate``;
 * the parameter-gradient reductions over slots: ``ow_bwd_param_reduce64`` from the d = 64 fused
   kernel's P_u, P_v, dW' (recomputing U', V', dZ and the gate), ``ow_bwd_param_reduce128`` over the d = 128 channel
-  kernels' slot-major ones (fp32 batched GEMMs for the fp32 path), and every per-workgroup fp32
+  kernels' slot-major ones, and every per-workgroup fp32
   partial summed by ``ow_sum_rows`` in a fixed order.
 
 Gradients are formed for the folded operands the forward evaluates (B_u'' = -log2(e) w B_u,
@@ -315,6 +317,9 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
             _native.check(lib.ow_rms_scale(x.data_ptr(), rscale.data_ptr(), n_rows, plan.channels, eps, code,
                                            stream), "ow_rms_scale")
 
+        if dtype == torch.float32 and lib.ow_bwd_x3_packed_bytes(q_c, d, rd):
+            return _backward_x3(lib, grad, grad_delta, x, rscale, nw, gm, au, av, ao, ws, wdtype, plan, tok, ch, oplan,
+                                g_all, residual, stream), g_all, None
         g = torch.empty(n_rows, plan.channels, dtype=dtype, device=dev)  # fully written: no clearing
         # Routed tiles of X' = x r and of dY.
         xt = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
@@ -385,6 +390,56 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
 
     g_a.copy_(torch.stack([g_au.reshape(256), g_av.reshape(256), g_ao.reshape(256)]))
     return dx, g_all, None
+
+
+def _backward_x3(lib, grad: Tensor, grad_delta: Tensor, x: Tensor, rscale: Tensor | None, nw: Tensor | None, gm: Tensor,
+                 au: Tensor, av: Tensor, ao: Tensor, ws: list[Tensor], wdtype: torch.dtype, plan: RoutePlan, tok: Tensor,
+                 ch: Tensor, oplan, g_all: Tensor, residual: bool, stream: int) -> Tensor:
+    """The fp32 pass on the three-part kernels (``ow_bwd_channel_x3``, ``ow_bwd_param_reduce_x3``):
+    dx, and the parameter gradients into ``g_all`` (layout of ``_cast_grads``)."""
+    dev = x.device
+    batch = x.shape[0]
+    q_c, d, rd = ws[0].shape
+    q_s = plan.token_indices.shape[0]
+    slots = batch * q_s * 16
+    n_tok, channels = plan.height * plan.width, plan.channels
+    n_rows = batch * n_tok
+    dx = torch.empty_like(x)
+    if n_rows == 0:
+        g_all.zero_()
+        return dx
+    f32 = _DTYPE_CODE[torch.float32]
+    nd, nr, nb = q_c * slots * d, q_c * slots * rd, q_c * d * rd
+    packed_bytes = lib.ow_bwd_x3_packed_bytes(q_c, d, rd)
+    n_part = lib.ow_bwd_channel_x3_partials(slots, q_c)
+    ranges = lib.ow_bwd_param_reduce_x3_ranges(slots, q_c)
+    # One buffer: xt, dyt, P_u, P_v, dW', Z, dU', dV', g, the partial sums, the folded-weight
+    # gradients and the packed weights (every size but g's and the last a multiple of 16 bytes).
+    sizes = [nd] * 5 + [nr] * 3 + [768 * n_part, ranges * 3 * nb, 3 * nb, packed_bytes // 4, n_rows * channels]
+    work = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
+    ptr = [work.data_ptr()]
+    for n in sizes[:-1]:
+        ptr.append(ptr[-1] + 4 * n)
+    xt, dyt, pu, pv, dw, z, du, dv, part_a, part_b, d_b, packed, g = ptr
+    rs, nwp = (t.data_ptr() if t is not None else None for t in (rscale, nw))
+    w_args = (*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype], nwp, gm.data_ptr(), ch.data_ptr(), channels, q_c, d, rd)
+    check = _native.check
+    check(lib.ow_bwd_gather(x.data_ptr(), grad_delta.data_ptr(), rs, tok.data_ptr(), ch.data_ptr(), ctypes.byref(oplan),
+                            batch, f32, xt, dyt, stream), "ow_bwd_gather")
+    check(lib.ow_pack_bwd_x3(*w_args, packed, packed_bytes, stream), "ow_pack_bwd_x3")
+    check(lib.ow_bwd_channel_x3(xt, dyt, au.data_ptr(), av.data_ptr(), ao.data_ptr(), packed, packed_bytes, pu, pv, dw,
+                                z, du, dv, tok.data_ptr(), ch.data_ptr(), slots, n_tok, channels, q_s, q_c, d, rd, g,
+                                part_a, n_part, g_all.data_ptr(), stream), "ow_bwd_channel_x3")
+    check(lib.ow_bwd_param_reduce_x3(pu, pv, dw, z, du, dv, part_b, ranges, slots, q_c, d, rd, stream),
+          "ow_bwd_param_reduce_x3")
+    check(lib.ow_sum_rows(part_b, ranges, 3 * nb, d_b, stream), "ow_sum_rows")
+    check(lib.ow_bwd_rmsnorm(x.data_ptr(), g, rs, grad.data_ptr(), dx.data_ptr(), n_rows, channels, int(residual), f32,
+                             stream), "ow_bwd_rmsnorm")
+    out = g_all.data_ptr() + 4 * 768
+    gamma_out = out + 4 * 3 * nb
+    check(lib.ow_bwd_params(*w_args, d_b, d_b + 4 * nb, d_b + 8 * nb, out, out + 4 * nb, out + 8 * nb, gamma_out,
+                            gamma_out + 4 * channels if nw is not None else None, stream), "ow_bwd_params")
+    return dx
 
 
 def _cast_group(ts: tuple[Tensor, ...], dtypes: tuple[torch.dtype, ...]) -> tuple[Tensor, ...]:

@@ -62,4 +62,15 @@ __device__ __forceinline__ f32x16 x3_mma(const X3& a, const X3& b, f32x16 c) {
   return BF16::mma32(a.p[0], b.p[0], c);
 }
 
+// The same with the five smaller products in a sum of their own: one rounding at the size of the
+// sum per product instead of six (long chains, where those roundings are the error).
+__device__ __forceinline__ void x3_mma_apart(const X3& a, const X3& b, f32x16& hi, f32x16& lo) {
+  lo = BF16::mma32(a.p[2], b.p[0], lo);
+  lo = BF16::mma32(a.p[1], b.p[1], lo);
+  lo = BF16::mma32(a.p[0], b.p[2], lo);
+  lo = BF16::mma32(a.p[1], b.p[0], lo);
+  lo = BF16::mma32(a.p[0], b.p[1], lo);
+  hi = BF16::mma32(a.p[0], b.p[0], hi);
+}
+
 }  // namespace ow
