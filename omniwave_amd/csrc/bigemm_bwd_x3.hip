@@ -13,9 +13,9 @@
 // the operands of the first three products take 288 registers and the sums of the second three
 // 192.  Each value that crosses is written once and read twice (chan2_x3, reduce_x3).
 //
-// 28x28x256, B = 32 (100,352 slots of 64 channels): 82 + 74 + 51 us, 3.4 / 3.1 / 4.5 TB/s, where
+// 28x28x256, B = 32 (100,352 slots of 64 channels): 80 + 72 + 51 us, 3.5 / 3.2 / 4.5 TB/s, where
 // fp32 products of the library around a gate kernel, token mixings, per-tile outer products and
-// the scatter took 460; the whole step 640 -> 340 us.  Errors against 64 bits over 4x4 to 56x56
+// the scatter took 460; the whole step 640 -> 330 us.  Errors against 64 bits over 4x4 to 56x56
 // images: dx 1.7e-7 (2.6e-7 before), weights' 4.2e-7 (7.2e-7), token matrices' 4.3e-7 (5.5e-7).
 #include <hip/hip_runtime.h>
 
@@ -217,12 +217,12 @@ chan_x3_kernel(ChanX3Args a) {
     }
   };
   {
-    float raw[MB][16];
-    load_rows(rows.of(a.xt, D), raw);
-    token_side(raw, token_operand(a.a_u, false, l32, hh), rows.of(a.pu, D), P[0]);
-    token_side(raw, token_operand(a.a_v, false, l32, hh), rows.of(a.pv, D), P[1]);
-    load_rows(rows.of(a.dyt, D), raw);
-    token_side(raw, token_operand(a.a_o, true, l32, hh), rows.of(a.dw, D), P[2]);
+    float x[MB][16], y[MB][16];  // all of a lane's loads in flight at once
+    load_rows(rows.of(a.xt, D), x);
+    load_rows(rows.of(a.dyt, D), y);
+    token_side(x, token_operand(a.a_u, false, l32, hh), rows.of(a.pu, D), P[0]);
+    token_side(x, token_operand(a.a_v, false, l32, hh), rows.of(a.pv, D), P[1]);
+    token_side(y, token_operand(a.a_o, true, l32, hh), rows.of(a.dw, D), P[2]);
   }
   const __amdgpu_buffer_rsrc_t rz = rows.of(a.z, a.rd), rdu = rows.of(a.du, a.rd), rdv = rows.of(a.dv, a.rd);
   const uint32_t wide = static_cast<uint32_t>(l32 * a.rd + 4 * hh) * 4u;

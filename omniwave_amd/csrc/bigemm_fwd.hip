@@ -1524,6 +1524,7 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
   const bool persist = ow::fwd_uses_persist(x, out, plan, rd, dtype, flags, batch);
   const bool split = persist && ow::fwd_uses_split(plan, q_s, q_c, flags, batch);
   float* scale = nullptr;
+  bool x3_norm = false;  // the fp32 kernel forms the scales itself
   // scale_out (ow_bigemm_fwd_scales): the row scales go to the caller's buffer where the launch
   // forms them in one place (the statistics pass, or the 16-token kernel below).
   const bool want_scales = scale_out && norm && !out_rows;
@@ -1536,15 +1537,16 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
                    need);
       scale = static_cast<float*>(workspace);
     }
-    if (wave16 || (split && ow::split_inline(q_c))) {
+    x3_norm = x3 && !want_scales && ow::x3_forms_scales(batch, q_s, q_c);
+    if (wave16 || x3_norm || (split && ow::split_inline(q_c))) {
       scale = nullptr;  // the kernel forms the scales itself
     } else if (int rc = ow_rms_scale(x, scale, static_cast<int64_t>(batch) * n, c, eps, dtype, stream)) return rc;
     if (want_scales && scale) *scale_written = 1;
   }
 
   if (x3) {
-    if (int rc = ow::launch_fwd_x3(static_cast<const float*>(x), static_cast<float*>(out), scale, packed, token_index,
-                                   channel_index, batch, n, c, q_s, q_c, d, rd, (flags & OW_FUSE_RESIDUAL) ? 1 : 0,
+    if (int rc = ow::launch_fwd_x3(static_cast<const float*>(x), static_cast<float*>(out), scale, x3_norm, eps, packed,
+                                   token_index, channel_index, batch, n, c, q_s, q_c, d, rd, (flags & OW_FUSE_RESIDUAL) ? 1 : 0,
                                    drop_scale, s))
       return rc;
     ow::clear_error();

@@ -108,13 +108,15 @@ __global__ void __launch_bounds__(256) pack_x3_kernel(PackX3Args p) {
 struct X3Args {
   const float* x;
   float* out;
-  const float* row_scale;  // NULL: no RMSNorm
+  const float* row_scale;  // NULL: no RMSNorm, or the kernel forms the scales (norm)
   const uint8_t* packed;
   const int32_t* tok;
   const int32_t* chan;
   const float* drop_scale;  // [batch] per-image multiplier of delta (drop-path); NULL: none
   int32_t batch, n_tok, channels, q_s, q_c, residual;
   int32_t n_groups;  // batch * q_s token groups
+  int32_t norm;      // S = 4: form the RMSNorm scales here
+  float eps;
 };
 
 // S waves share a pair, each with an S-th of the expanded dimension (W summed over them at the
@@ -217,6 +219,24 @@ bigemm_fwd_x3_kernel(X3Args a) {
   };
   const bool g0 = (lane & 16) == 0;
   __syncthreads();
+  if constexpr (S == 4) {
+    if (a.norm) {  // eight lanes a row, 128 bytes of it a step (a ragged row's last vector is cut off)
+      const uint32_t base = s_off[0][tid >> 3];
+      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+      for (int c = 4 * (tid & 7); c < a.channels; c += 32) {
+        const f32x4 v = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, static_cast<int>(base + 4u * static_cast<uint32_t>(c)), 0, 0));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] = c + k < a.channels ? fmaf(v[k], v[k], acc[k]) : acc[k];
+      }
+      float sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+      for (int m = 4; m > 0; m >>= 1) sum += __shfl_xor(sum, m);
+      if ((tid & 7) == 0) s_scale[0][tid >> 3] = base == kOffOut ? 0.0f : 1.0f / sqrtf(sum / static_cast<float>(a.channels) + a.eps);
+      __syncthreads();
+    }
+  }
 
   auto channel = [&](int mb) -> uint32_t {  // byte offset of the lane's channel of a 32-channel block
     const int32_t ch = a.chan[q * D + 32 * mb + l32];
@@ -506,6 +526,16 @@ bigemm_fwd_x3_kernel(X3Args a) {
   }
 }
 
+// With fewer units than four per CU the waves of a workgroup share one pair (or two) and its
+// expanded dimension: a workgroup still holds one CU, and each unit is done sooner.  Measured on
+// an earlier form of the loop at 14x14x512: B = 8 (208 units) 24 us split in four, 30 in two, 42
+// whole; B = 16 (416) 41, 33, 44; B = 32 (832) 77, 60, 49.  d = 64 crosses at the same counts
+// (28x28x256, 196 units: 12.8, 13.6, 17.9; 392: 21, 15, 18; 784: 38, 21, 20).
+int x3_split(int64_t units) {
+  const int64_t cus = device_cus();
+  return units <= cus ? 4 : units <= 2 * cus ? 2 : 1;
+}
+
 template <int D, int RD>
 int launch_x3(const X3Args& a, int32_t n_pairs, int split, hipStream_t stream) {
   const unsigned grid = static_cast<unsigned>(static_cast<int64_t>((n_pairs + 4 / split - 1) / (4 / split)) * a.q_c);
@@ -539,24 +569,25 @@ int pack_weights_x3(const void* a_u, const void* a_v, const void* a_o, const voi
   return hip_status(hipGetLastError(), "pack_x3_kernel launch");
 }
 
-int launch_fwd_x3(const float* x, float* out, const float* row_scale, const void* packed, const int32_t* tok,
-                  const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s, int32_t q_c,
-                  int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream) {
+// Split in four, a workgroup holds one pair and forms its rows' RMSNorm scales itself: 32 rows by
+// 256 threads, read by the q_c workgroups of the pair from L2, against a launch of its own.
+// 14x14x512, B = 8: 2.4 us more in this kernel against a pass of 4.3 and the gap before it; with
+// whole pairs per wave four times the rows would wait for their reads, beside a pass of 6 us in 40.
+bool x3_forms_scales(int32_t batch, int32_t q_s, int32_t q_c) {
+  return x3_split((static_cast<int64_t>(batch) * q_s + 1) / 2 * q_c) == 4;
+}
+
+int launch_fwd_x3(const float* x, float* out, const float* row_scale, bool norm, float eps, const void* packed,
+                  const int32_t* tok, const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s,
+                  int32_t q_c, int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream) {
   const int64_t groups = static_cast<int64_t>(batch) * q_s;
   if (groups >= (int64_t(1) << 31)) return fail(OW_ERR_UNSUPPORTED, "batch * token groups must be below 2^31");
   X3Args a{x, out, row_scale, static_cast<const uint8_t*>(packed), tok, chan, drop_scale, batch, n_tok, channels,
-           q_s, q_c, residual, static_cast<int32_t>(groups)};
+           q_s, q_c, residual, static_cast<int32_t>(groups), norm ? 1 : 0, eps};
   const int32_t n_pairs = static_cast<int32_t>((groups + 1) / 2);
   // A workgroup's offsets start at its first image: the images its 8 token groups can span.
   if (!x3_fits(n_tok, channels, q_s)) return fail(OW_ERR_UNSUPPORTED, "images too large for 32-bit offsets");
-  const int64_t units = static_cast<int64_t>(n_pairs) * q_c;
-  const int64_t cus = device_cus();
-  // With fewer units than four per CU the waves of a workgroup share one pair (or two) and its
-  // expanded dimension: a workgroup still holds one CU, and each unit is done sooner.  Measured on
-  // an earlier form of the loop at 14x14x512: B = 8 (208 units) 24 us split in four, 30 in two, 42
-  // whole; B = 16 (416) 41, 33, 44; B = 32 (832) 77, 60, 49.  d = 64 crosses at the same counts
-  // (28x28x256, 196 units: 12.8, 13.6, 17.9; 392: 21, 15, 18; 784: 38, 21, 20).
-  const int split = units <= cus ? 4 : units <= 2 * cus ? 2 : 1;
+  const int split = x3_split(static_cast<int64_t>(n_pairs) * q_c);
   if (d == 64 && rd == 128) return launch_x3<64, 128>(a, n_pairs, split, stream);
   if (d == 64 && rd == 256) return launch_x3<64, 256>(a, n_pairs, split, stream);
   if (d == 128 && rd == 128) return launch_x3<128, 128>(a, n_pairs, split, stream);
