@@ -457,11 +457,12 @@ int ow_bwd_param_reduce128(const void* pu, const void* pv, const void* dw, const
                            int32_t dtype, void* stream);
 
 /* The fp32 backward's channel side on the bf16 matrix cores, every fp32 operand as three bf16
- * parts and a product as the six part products above 2^-24 (replaces ow_tile_mix, ow_tile_outer,
+ * parts and a product as the six part products above 2^-24 (replaces ow_bwd_gather, ow_tile_mix, ow_tile_outer,
  * ow_bwd_gate, ow_bwd_scatter and the channel GEMMs; the reference's fp32 autograd recompute,
  * omniweave/ops/triton.py:256-292).  ow_pack_bwd_x3: the folded weights (as ow_fold_weights; formed
  * in fp64) in parts, ow_bwd_x3_packed_bytes(q_c, d, rd) bytes (0: unsupported shape).
- * ow_bwd_channel_x3: from the fp32 tiles X', dY ([q_c][slots][d], ow_bwd_gather), P_u, P_v, dW'
+ * ow_bwd_channel_x3: from x, dy [rows][channels] and the row scales (NULL: 1), read through the
+ * tables (images within 32-bit offsets: ow_bwd_x3_fits), slots = batch * q_s * 16: P_u, P_v, dW'
  * ([q_c][slots][d]) and Z, dU', dV' ([q_c][slots][rd]) as ow_bwd_channel, then dX' written to
  * g [rows][channels] at its routed place (every element once) and the token-matrix gradients
  * dA_u, dA_v, dA_o to d_a [3][256] (partial: workspace of n_partial =
@@ -473,10 +474,11 @@ size_t ow_bwd_x3_packed_bytes(int32_t q_c, int32_t d, int32_t rd);
 int ow_pack_bwd_x3(const void* b_u, const void* b_v, const void* b_o, int32_t weight_dtype, const float* norm_weight,
                    const float* gamma, const int32_t* channel_index, int32_t channels, int32_t q_c, int32_t d,
                    int32_t rd, void* packed, size_t packed_bytes, void* stream);
+int ow_bwd_x3_fits(int32_t n_tok, int32_t channels, int32_t q_s);
 int64_t ow_bwd_channel_x3_partials(int64_t slots, int32_t q_c);
-int ow_bwd_channel_x3(const float* xt, const float* dyt, const float* a_u, const float* a_v, const float* a_o,
+int ow_bwd_channel_x3(const float* x, const float* dy, const float* rscale, const float* a_u, const float* a_v, const float* a_o,
                       const void* packed, size_t packed_bytes, float* pu, float* pv, float* dw, float* z, float* du,
-                      float* dv, const int32_t* token_index, const int32_t* channel_index, int64_t slots, int32_t n_tok,
+                      float* dv, const int32_t* token_index, const int32_t* channel_index, int32_t batch, int32_t n_tok,
                       int32_t channels, int32_t q_s, int32_t q_c, int32_t d, int32_t rd, float* g, float* partial,
                       int64_t n_partial, float* d_a, void* stream);
 int64_t ow_bwd_param_reduce_x3_ranges(int64_t slots, int32_t q_c);

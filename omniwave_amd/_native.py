@@ -214,10 +214,11 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 3 + [ctypes.c_int32] + [ctypes.c_void_p] * 3 + [ctypes.c_int32] * 4
         + [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p],
     ),
+    "ow_bwd_x3_fits": (ctypes.c_int, [ctypes.c_int32] * 3),
     "ow_bwd_channel_x3_partials": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32]),
     "ow_bwd_channel_x3": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 6 + [ctypes.c_size_t] + [ctypes.c_void_p] * 8 + [ctypes.c_int64] + [ctypes.c_int32] * 6
+        [ctypes.c_void_p] * 7 + [ctypes.c_size_t] + [ctypes.c_void_p] * 8 + [ctypes.c_int32] * 7
         + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p],
     ),
     "ow_bwd_param_reduce_x3_ranges": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32]),

@@ -317,9 +317,10 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
             _native.check(lib.ow_rms_scale(x.data_ptr(), rscale.data_ptr(), n_rows, plan.channels, eps, code,
                                            stream), "ow_rms_scale")
 
-        if dtype == torch.float32 and lib.ow_bwd_x3_packed_bytes(q_c, d, rd):
-            return _backward_x3(lib, grad, grad_delta, x, rscale, nw, gm, au, av, ao, ws, wdtype, plan, tok, ch, oplan,
-                                g_all, residual, stream), g_all, None
+        if (dtype == torch.float32 and lib.ow_bwd_x3_packed_bytes(q_c, d, rd)
+                and lib.ow_bwd_x3_fits(plan.height * plan.width, plan.channels, q_s)):
+            return _backward_x3(lib, grad, grad_delta, x, rscale, nw, gm, au, av, ao, ws, wdtype, plan, tok, ch, g_all,
+                                residual, stream), g_all, None
         g = torch.empty(n_rows, plan.channels, dtype=dtype, device=dev)  # fully written: no clearing
         # Routed tiles of X' = x r and of dY.
         xt = torch.empty(q_c, slots, d, dtype=dtype, device=dev)
@@ -394,7 +395,7 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
 
 def _backward_x3(lib, grad: Tensor, grad_delta: Tensor, x: Tensor, rscale: Tensor | None, nw: Tensor | None, gm: Tensor,
                  au: Tensor, av: Tensor, ao: Tensor, ws: list[Tensor], wdtype: torch.dtype, plan: RoutePlan, tok: Tensor,
-                 ch: Tensor, oplan, g_all: Tensor, residual: bool, stream: int) -> Tensor:
+                 ch: Tensor, g_all: Tensor, residual: bool, stream: int) -> Tensor:
     """The fp32 pass on the three-part kernels (``ow_bwd_channel_x3``, ``ow_bwd_param_reduce_x3``):
     dx, and the parameter gradients into ``g_all`` (layout of ``_cast_grads``)."""
     dev = x.device
@@ -413,22 +414,20 @@ def _backward_x3(lib, grad: Tensor, grad_delta: Tensor, x: Tensor, rscale: Tenso
     packed_bytes = lib.ow_bwd_x3_packed_bytes(q_c, d, rd)
     n_part = lib.ow_bwd_channel_x3_partials(slots, q_c)
     ranges = lib.ow_bwd_param_reduce_x3_ranges(slots, q_c)
-    # One buffer: xt, dyt, P_u, P_v, dW', Z, dU', dV', g, the partial sums, the folded-weight
+    # One buffer: P_u, P_v, dW', Z, dU', dV', g, the partial sums, the folded-weight
     # gradients and the packed weights (every size but g's and the last a multiple of 16 bytes).
-    sizes = [nd] * 5 + [nr] * 3 + [768 * n_part, ranges * 3 * nb, 3 * nb, packed_bytes // 4, n_rows * channels]
+    sizes = [nd] * 3 + [nr] * 3 + [768 * n_part, ranges * 3 * nb, 3 * nb, packed_bytes // 4, n_rows * channels]
     work = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
     ptr = [work.data_ptr()]
     for n in sizes[:-1]:
         ptr.append(ptr[-1] + 4 * n)
-    xt, dyt, pu, pv, dw, z, du, dv, part_a, part_b, d_b, packed, g = ptr
+    pu, pv, dw, z, du, dv, part_a, part_b, d_b, packed, g = ptr
     rs, nwp = (t.data_ptr() if t is not None else None for t in (rscale, nw))
     w_args = (*[w.data_ptr() for w in ws], _DTYPE_CODE[wdtype], nwp, gm.data_ptr(), ch.data_ptr(), channels, q_c, d, rd)
     check = _native.check
-    check(lib.ow_bwd_gather(x.data_ptr(), grad_delta.data_ptr(), rs, tok.data_ptr(), ch.data_ptr(), ctypes.byref(oplan),
-                            batch, f32, xt, dyt, stream), "ow_bwd_gather")
     check(lib.ow_pack_bwd_x3(*w_args, packed, packed_bytes, stream), "ow_pack_bwd_x3")
-    check(lib.ow_bwd_channel_x3(xt, dyt, au.data_ptr(), av.data_ptr(), ao.data_ptr(), packed, packed_bytes, pu, pv, dw,
-                                z, du, dv, tok.data_ptr(), ch.data_ptr(), slots, n_tok, channels, q_s, q_c, d, rd, g,
+    check(lib.ow_bwd_channel_x3(x.data_ptr(), grad_delta.data_ptr(), rs, au.data_ptr(), av.data_ptr(), ao.data_ptr(), packed, packed_bytes, pu, pv, dw,
+                                z, du, dv, tok.data_ptr(), ch.data_ptr(), batch, n_tok, channels, q_s, q_c, d, rd, g,
                                 part_a, n_part, g_all.data_ptr(), stream), "ow_bwd_channel_x3")
     check(lib.ow_bwd_param_reduce_x3(pu, pv, dw, z, du, dv, part_b, ranges, slots, q_c, d, rd, stream),
           "ow_bwd_param_reduce_x3")

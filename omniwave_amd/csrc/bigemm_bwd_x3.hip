@@ -1,6 +1,6 @@
 // fp32 backward of the channel side on the bf16 matrix cores (three-part operands, ow_x3.h): the
-// gradients of omniweave/ops/reference.py:120-173 (autograd there) in three kernels over the
-// routed tiles X', dY of ow_bwd_gather, for d, rd as the forward.
+// gradients of omniweave/ops/reference.py:120-173 (autograd there) in three kernels,
+// for d, rd as the forward.  x r and dy are read where they lie, through the token and channel tables.
 //
 //   chan_x3     P_u = A_u X', P_v = A_v X', dW' = A_o^T dY, then per 32-row chunk of the expanded
 //               dimension U', V', dZ and the gate backward: Z, dU', dV'
@@ -13,10 +13,11 @@
 // the operands of the first three products take 288 registers and the sums of the second three
 // 192.  Each value that crosses is written once and read twice (chan2_x3, reduce_x3).
 //
-// 28x28x256, B = 32 (100,352 slots of 64 channels): 80 + 72 + 51 us, 3.5 / 3.2 / 4.5 TB/s, where
-// fp32 products of the library around a gate kernel, token mixings, per-tile outer products and
-// the scatter took 460; the whole step 640 -> 330 us.  Errors against 64 bits over 4x4 to 56x56
-// images: dx 1.7e-7 (2.6e-7 before), weights' 4.2e-7 (7.2e-7), token matrices' 4.3e-7 (5.5e-7).
+// 28x28x256, B = 32 (100,352 slots of 64 channels): 81 + 78 + 52 us, where fp32 products of the
+// library around a gate kernel, gather, token mixings, per-tile outer products and the scatter took
+// 485; the whole step 640 -> 310 us.  With routed tiles X', dY written by a gather kernel first (27
+// us) the three took 80 + 72 + 51.  Errors against 64 bits over 4x4 to 56x56 images: dx 1.7e-7
+// (2.6e-7 before), weights' 4.3e-7 (7.2e-7), token matrices' 4.3e-7 (5.5e-7).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -97,8 +98,9 @@ __global__ void __launch_bounds__(kThreads) pack_bwd_x3_kernel(PackBwdX3Args p) 
 }
 
 struct ChanX3Args {
-  const float* xt;
-  const float* dyt;
+  const float* x;
+  const float* dy;
+  const float* rscale;  // NULL: 1
   const float* a_u;
   const float* a_v;
   const float* a_o;
@@ -114,7 +116,7 @@ struct ChanX3Args {
   const int32_t* tok;
   const int32_t* chan;
   int64_t slots;
-  int32_t q_c, rd, n_tok, channels, q_s;
+  int32_t q_c, rd, n_tok, channels, q_s, batch;
 };
 
 // Row l32 % 16 of a token matrix (or of its transpose), 8 entries in the K order of the pair scheme.
@@ -155,6 +157,47 @@ __device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t r, uint32_t off, c
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), r, static_cast<int>(off), 0, 0);
 }
 
+// Routed x and dy: a buffer from the first image of the workgroup's pairs on, of at most 1 GiB; a pad
+// slot's row offset lies at 2 GiB and a pad channel's at 1 GiB, so what either asks for reads as zero
+// without a branch.
+constexpr int64_t kSpan = int64_t(1) << 30;
+struct Routed {
+  int64_t img0;
+  __device__ __forceinline__ Routed(const ChanX3Args& a, int64_t pair0) : img0(2 * pair0 / a.q_s) {}
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t of(const float* p, const ChanX3Args& a) const {
+    const int64_t img = static_cast<int64_t>(a.n_tok) * a.channels, left = (a.batch - img0) * img * 4;
+    return buffer_rsrc(p + img0 * img, static_cast<uint32_t>(left < kSpan ? left : kSpan));
+  }
+};
+// The workgroup's 128 slots: byte offset of the row, row number (-1: pad) and RMSNorm scale.
+struct SlotTables {
+  uint32_t off[4][32];
+  int32_t row[4][32];
+  float scale[4][32];
+  __device__ __forceinline__ void fill(const ChanX3Args& a, int64_t pair0, int64_t img0, int t) {
+    const int64_t slot = 32 * pair0 + t;
+    uint32_t o = kOffOut;
+    int32_t r = -1;
+    float s = 0.0f;
+    if (slot < a.slots) {
+      const int64_t b = (slot >> 4) / a.q_s;
+      const int32_t tk = a.tok[((slot >> 4) - b * a.q_s) * kG + (slot & 15)];
+      if (tk >= 0 && tk < a.n_tok) {
+        o = static_cast<uint32_t>((b - img0) * a.n_tok + tk) * static_cast<uint32_t>(a.channels) * 4u;
+        r = static_cast<int32_t>(b * a.n_tok + tk);
+        s = a.rscale ? a.rscale[r] : 1.0f;
+      }
+    }
+    off[t >> 5][t & 31] = o;
+    row[t >> 5][t & 31] = r;
+    scale[t >> 5][t & 31] = s;
+  }
+};
+__device__ __forceinline__ uint32_t channel_offset(const ChanX3Args& a, int64_t i) {
+  const int32_t ch = a.chan[i];
+  return ch >= 0 && ch < a.channels ? 4u * static_cast<uint32_t>(ch) : static_cast<uint32_t>(kSpan);
+}
+
 // The weight chunks of one group and phase through two LDS buffers: every wave copies a quarter.
 template <int KS>
 struct ChunkRing {
@@ -172,6 +215,11 @@ struct ChunkRing {
 };
 __device__ __forceinline__ X3 ring_frag(const u32x4* p) { return X3{{p[0], p[64], p[128]}}; }
 
+// Workgroups are dispatched round-robin over the 8 XCDs: the q_c groups of one block of pairs lie 8
+// apart, on one XCD, whose L2 then serves the rows that interleaved groups share (28x28x256 radix,
+// B = 32, the whole step 380 -> 345 us; 7x7x1024 radix, B = 64, 370 -> 340; contiguous groups the
+// same or a little less).
+//
 // Four waves, each a 32-slot pair, share a group's weight chunks (36 KB at d = 64, 72 KB at
 // d = 128) through two LDS buffers, one barrier a chunk.  A chunk's copies have its predecessor's
 // products to land in, and its stores its successor's.  Bound by memory: the rows are read once
@@ -183,24 +231,31 @@ chan_x3_kernel(ChanX3Args a) {
   constexpr int KS = D / 16, MB = D / 32;
   using Ring = ChunkRing<KS>;
   __shared__ __attribute__((aligned(16))) u32x4 ring[2][Ring::FR * 64];
+  __shared__ __attribute__((aligned(16))) SlotTables tab;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = static_cast<int>(blockIdx.x) % a.q_c;
-  const PairRows rows = pair_rows(a.slots, q, static_cast<int64_t>(blockIdx.x) / a.q_c * 4 + wave);
+  const int q = static_cast<int>(blockIdx.x / 8) % a.q_c;
+  const int64_t block = static_cast<int64_t>(blockIdx.x) / (8 * a.q_c) * 8 + blockIdx.x % 8, pair0 = 4 * block;
+  if (32 * pair0 >= a.slots) return;
+  const PairRows rows = pair_rows(a.slots, q, pair0 + wave);
+  const Routed routed(a, pair0);
   const int ne = a.rd / 32;
   const Ring copier{a.packed + static_cast<int64_t>(q) * 2 * ne * Ring::FR * 1024, lds_addr(&ring[0][0]),
                     16u * static_cast<uint32_t>(lane), wave};
   copier.copy(0, 0);
 
+  if (tid < 128) tab.fill(a, pair0, routed.img0, tid);
+  __syncthreads();
   const bool g0 = (lane & 16) == 0;
   X3 P[3][KS];  // P_u, P_v, dW' as K-step operands
   const f32x16 zero = {};
   auto load_rows = [&](const __amdgpu_buffer_rsrc_t& r, float(&v)[MB][16]) {
 #pragma unroll
-    for (int cb = 0; cb < MB; ++cb)
+    for (int cb = 0; cb < MB; ++cb) {
+      const uint32_t ch = channel_offset(a, q * D + 32 * cb + l32);
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        v[cb][i] = load1(r, static_cast<uint32_t>(pair_token_row(i, hh) * D + 32 * cb + l32) * 4u);
+      for (int i = 0; i < 16; ++i) v[cb][i] = load1(r, tab.off[wave][pair_token_row(i, hh)] + ch);
+    }
   };
   const uint32_t own = static_cast<uint32_t>(l32 * D + 4 * hh) * 4u;
   auto token_side = [&](const float(&raw)[MB][16], const X3& m, const __amdgpu_buffer_rsrc_t& out, X3(&op)[KS]) {
@@ -218,8 +273,14 @@ chan_x3_kernel(ChanX3Args a) {
   };
   {
     float x[MB][16], y[MB][16];  // all of a lane's loads in flight at once
-    load_rows(rows.of(a.xt, D), x);
-    load_rows(rows.of(a.dyt, D), y);
+    load_rows(routed.of(a.x, a), x);
+    load_rows(routed.of(a.dy, a), y);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float r = tab.scale[wave][pair_token_row(i, hh)];
+#pragma unroll
+      for (int cb = 0; cb < MB; ++cb) x[cb][i] *= r;
+    }
     token_side(x, token_operand(a.a_u, false, l32, hh), rows.of(a.pu, D), P[0]);
     token_side(x, token_operand(a.a_v, false, l32, hh), rows.of(a.pv, D), P[1]);
     token_side(y, token_operand(a.a_o, true, l32, hh), rows.of(a.dw, D), P[2]);
@@ -268,27 +329,20 @@ chan2_x3_kernel(ChanX3Args a) {
   constexpr int KS = D / 16, MB = D / 32, LD = 36;
   using Ring = ChunkRing<KS>;
   __shared__ __attribute__((aligned(16))) u32x4 ring[2][Ring::FR * 64];
-  __shared__ int32_t s_row[4][32];
+  __shared__ __attribute__((aligned(16))) SlotTables tab;
   static_assert(sizeof(ring) >= 4 * (32 * LD + 768) * sizeof(float), "the epilogue's LDS fits the ring");
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = static_cast<int>(blockIdx.x) % a.q_c;
-  const int64_t pair0 = static_cast<int64_t>(blockIdx.x) / a.q_c * 4;
+  const int q = static_cast<int>(blockIdx.x / 8) % a.q_c;
+  const int64_t block = static_cast<int64_t>(blockIdx.x) / (8 * a.q_c) * 8 + blockIdx.x % 8, pair0 = 4 * block;
+  if (32 * pair0 >= a.slots) return;
   const PairRows rows = pair_rows(a.slots, q, pair0 + wave);
   const int ne = a.rd / 32;
   const Ring copier{a.packed + (static_cast<int64_t>(q) * 2 + 1) * ne * Ring::FR * 1024, lds_addr(&ring[0][0]),
                     16u * static_cast<uint32_t>(lane), wave};
   copier.copy(0, 0);
-  if (tid < 128) {
-    const int64_t slot = 32 * pair0 + tid;
-    int32_t row = -1;
-    if (slot < a.slots) {
-      const int64_t b = (slot >> 4) / a.q_s;
-      const int32_t tk = a.tok[((slot >> 4) - b * a.q_s) * kG + (slot & 15)];
-      if (tk >= 0 && tk < a.n_tok) row = static_cast<int32_t>(b * a.n_tok + tk);
-    }
-    s_row[tid >> 5][tid & 31] = row;
-  }
+  const Routed routed(a, pair0);
+  if (tid < 128) tab.fill(a, pair0, routed.img0, tid);
 
   const float* src[3] = {a.du, a.dv, a.z};
   __amdgpu_buffer_rsrc_t r[3] = {rows.of(src[0], a.rd), rows.of(src[1], a.rd), rows.of(src[2], a.rd)};
@@ -328,28 +382,52 @@ chan2_x3_kernel(ChanX3Args a) {
 
   // dA_u = dP_u X'^T, dA_v = dP_v X'^T, dA_o = dY W'^T: 32x32 products of the pair's slots, of which
   // the two 16x16 blocks on the diagonal are its tiles.
-  f32x16 da[3];
-  {
-    const __amdgpu_buffer_rsrc_t rx = rows.of(a.xt, D), ry = rows.of(a.dyt, D);
-    const uint32_t own = static_cast<uint32_t>(l32 * D + 4 * hh) * 4u;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      f32x16 hi = zero, lo = zero;
-#pragma unroll
-      for (int f = 0; f < KS; ++f) {
-        const f32x4 v0 = load4(m < 2 ? rx : ry, own + 64u * f), v1 = load4(m < 2 ? rx : ry, own + 64u * f + 32u);
-        const X3 t = x3_split8([&](int j) { return j < 4 ? v0[j & 3] : v1[j & 3]; });
-        const X3 p = x3_kstep(acc[m][f >> 1], f & 1);
-        if (m < 2)
-          x3_mma_apart(p, t, hi, lo);
-        else
-          x3_mma_apart(t, p, hi, lo);
-      }
-      mfma_drain();
-      da[m] = hi + lo;
-    }
-  }
   float* scratch = reinterpret_cast<float*>(&ring[0][0]) + wave * 32 * LD;
+  f32x16 da[3];
+  // x r (or dy) of the pair with lane = channel, through LDS to lane = slot: the operand of K step f.
+  auto tiles = [&](const __amdgpu_buffer_rsrc_t& r, auto scaled, auto use) {
+    float v[MB][16];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const uint32_t ch = channel_offset(a, q * D + 32 * mb + l32);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[mb][i] = load1(r, tab.off[wave][pair_token_row(i, hh)] + ch);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = pair_token_row(i, hh);
+        scratch[t * LD + l32] = decltype(scaled)::value ? v[mb][i] * tab.scale[wave][t] : v[mb][i];
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const float* p = scratch + l32 * LD + 16 * s + 4 * hh;
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 8);
+        use(2 * mb + s, x3_split8([&](int j) { return j < 4 ? lo[j & 3] : hi[j & 3]; }));
+      }
+      wave_lds_sync();
+    }
+  };
+  {
+    f32x16 hi[2] = {zero, zero}, lo[2] = {zero, zero};
+    tiles(routed.of(a.x, a), std::integral_constant<bool, true>{}, [&](int f, const X3& t) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) x3_mma_apart(x3_kstep(acc[m][f >> 1], f & 1), t, hi[m], lo[m]);
+    });
+    mfma_drain();
+    da[0] = hi[0] + lo[0];
+    da[1] = hi[1] + lo[1];
+  }
+  {
+    f32x16 hi = zero, lo = zero;
+    tiles(routed.of(a.dy, a), std::integral_constant<bool, false>{}, [&](int f, const X3& t) {
+      x3_mma_apart(t, x3_kstep(acc[2][f >> 1], f & 1), hi, lo);
+    });
+    mfma_drain();
+    da[2] = hi + lo;
+  }
   float* sums = reinterpret_cast<float*>(&ring[0][0]) + 4 * 32 * LD;  // [wave][3][16][16]
 #pragma unroll
   for (int m = 0; m < 3; ++m)
@@ -364,7 +442,7 @@ chan2_x3_kernel(ChanX3Args a) {
   const bool g0 = (lane & 16) == 0;
   int32_t row[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) row[i] = s_row[wave][pair_token_row(i, hh)];
+  for (int i = 0; i < 16; ++i) row[i] = tab.row[wave][pair_token_row(i, hh)];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     f32x16 dx = zero;
@@ -393,7 +471,7 @@ chan2_x3_kernel(ChanX3Args a) {
   }
   __syncthreads();
   for (int i = tid; i < 768; i += kThreads)
-    a.partial[static_cast<int64_t>(blockIdx.x) * 768 + i] = (sums[i] + sums[768 + i]) + (sums[1536 + i] + sums[2304 + i]);
+    a.partial[(block * a.q_c + q) * 768 + i] = (sums[i] + sums[768 + i]) + (sums[1536 + i] + sums[2304 + i]);
 }
 
 // out[c] = the sum of partial[r][c] over the rows, c < 768, in fp64: 48 workgroups of 16 columns,
@@ -537,37 +615,45 @@ int ow_pack_bwd_x3(const void* b_u, const void* b_v, const void* b_o, int32_t we
   return OW_OK;
 }
 
+// A workgroup's offsets start at its first image: the images its 8 token groups can span.
+int ow_bwd_x3_fits(int32_t n_tok, int32_t channels, int32_t q_s) {
+  return q_s >= 1 && static_cast<int64_t>(8 / q_s + 2) * n_tok * channels * 4 < ow::kSpan;
+}
+
 int64_t ow_bwd_channel_x3_partials(int64_t slots, int32_t q_c) {
   return slots < 1 || q_c < 1 ? 0 : ow::blocks_of(slots, q_c);
 }
 
-int ow_bwd_channel_x3(const float* xt, const float* dyt, const float* a_u, const float* a_v, const float* a_o,
+int ow_bwd_channel_x3(const float* x, const float* dy, const float* rscale, const float* a_u, const float* a_v, const float* a_o,
                       const void* packed, size_t packed_bytes, float* pu, float* pv, float* dw, float* z, float* du,
-                      float* dv, const int32_t* token_index, const int32_t* channel_index, int64_t slots, int32_t n_tok,
+                      float* dv, const int32_t* token_index, const int32_t* channel_index, int32_t batch, int32_t n_tok,
                       int32_t channels, int32_t q_s, int32_t q_c, int32_t d, int32_t rd, float* g, float* partial,
                       int64_t n_partial, float* d_a, void* stream) {
+  const int64_t slots = static_cast<int64_t>(batch) * q_s * 16;
   OW_CHECK_SUPPORTED(ow::shape_ok(d, rd), "unsupported fp32 tile d=%d rd=%d", d, rd);
-  OW_CHECK_ARG(slots >= 0 && slots % 16 == 0, "slots must be a multiple of 16 (got %lld)", (long long)slots);
+  OW_CHECK_ARG(batch >= 0, "batch must be >= 0 (got %d)", batch);
   OW_CHECK_ARG(q_c >= 1 && q_s >= 1 && n_tok >= 1 && channels >= 1, "sizes must be positive");
   OW_CHECK_ARG(packed && packed_bytes >= ow_bwd_x3_packed_bytes(q_c, d, rd), "packed weights missing or too small");
+  OW_CHECK_SUPPORTED(ow_bwd_x3_fits(n_tok, channels, q_s), "images too large for 32-bit offsets");
   if (slots == 0) {
     ow::clear_error();
     return OW_OK;
   }
-  OW_CHECK_ARG(xt && dyt && a_u && a_v && a_o && pu && pv && dw && z && du && dv && token_index && channel_index && g &&
+  OW_CHECK_ARG(x && dy && a_u && a_v && a_o && pu && pv && dw && z && du && dv && token_index && channel_index && g &&
                    partial && d_a,
                "tensor pointer is NULL");
-  for (const void* p : {static_cast<const void*>(xt), static_cast<const void*>(dyt), packed, static_cast<const void*>(pu),
+  for (const void* p : {packed, static_cast<const void*>(pu),
                         static_cast<const void*>(pv), static_cast<const void*>(dw), static_cast<const void*>(z),
                         static_cast<const void*>(du), static_cast<const void*>(dv)})
     OW_CHECK_ARG(ow::aligned16(p), "tile buffers must be 16-byte aligned");
   const int64_t blocks = ow::blocks_of(slots, q_c);
   OW_CHECK_ARG(n_partial == blocks, "n_partial must be %lld", (long long)blocks);
-  OW_CHECK_SUPPORTED(blocks < (int64_t(1) << 31) && slots / 16 / q_s * n_tok < (int64_t(1) << 31),
+  OW_CHECK_SUPPORTED(blocks + 8 * q_c < (int64_t(1) << 31) && static_cast<int64_t>(batch) * n_tok < (int64_t(1) << 31),
                      "too many slots for one launch");
-  ow::ChanX3Args a{xt, dyt, a_u, a_v, a_o, static_cast<const uint8_t*>(packed), pu, pv, dw, z, du, dv, g, partial,
-                   token_index, channel_index, slots, q_c, rd, n_tok, channels, q_s};
-  const dim3 grid(static_cast<unsigned>(blocks)), threads(ow::kThreads);
+  ow::ChanX3Args a{x, dy, rscale, a_u, a_v, a_o, static_cast<const uint8_t*>(packed), pu, pv, dw, z, du, dv, g, partial,
+                   token_index, channel_index, slots, q_c, rd, n_tok, channels, q_s,
+                   batch};
+  const dim3 grid(static_cast<unsigned>((blocks / q_c + 7) / 8 * 8 * q_c)), threads(ow::kThreads);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (d == 64)
     hipLaunchKernelGGL(ow::chan_x3_kernel<64>, grid, threads, 0, s, a);
