@@ -1545,7 +1545,8 @@ static int bigemm_fwd_entry(const void* x, void* out, float eps, const void* pac
   }
 
   if (x3) {
-    if (int rc = ow::launch_fwd_x3(static_cast<const float*>(x), static_cast<float*>(out), scale, x3_norm, eps, packed,
+    if (int rc = ow::launch_fwd_x3(static_cast<const float*>(x), static_cast<float*>(out), scale, x3_norm, eps,
+                                   plan->radix_level > 0 && q_c > 1, packed,
                                    token_index, channel_index, batch, n, c, q_s, q_c, d, rd, (flags & OW_FUSE_RESIDUAL) ? 1 : 0,
                                    drop_scale, s))
       return rc;

@@ -117,6 +117,7 @@ struct X3Args {
   int32_t n_groups;  // batch * q_s token groups
   int32_t norm;      // S = 4: form the RMSNorm scales here
   float eps;
+  int32_t interleaved;  // radix channel groups
 };
 
 // S waves share a pair, each with an S-th of the expanded dimension (W summed over them at the
@@ -142,8 +143,14 @@ bigemm_fwd_x3_kernel(X3Args a) {
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int sub = wave % S, pl = wave / S;
-  const int q = static_cast<int>(blockIdx.x) % a.q_c;
-  const int pair0 = static_cast<int>(blockIdx.x) / a.q_c * NP;
+  // Interleaved groups share the lines of x and out: the q_c groups of one block of pairs lie 8
+  // workgroups apart, on one XCD (round-robin dispatch), whose L2 serves them (radix 1, B = 32:
+  // 28x28x256 77 -> 60 us, 14x14x512 59 -> 52).  Contiguous groups share nothing, and an XCD then
+  // reads one group's weights only where q_c divides 8 (the other order costs them 2 to 5%).
+  const int bid = static_cast<int>(blockIdx.x);
+  const int q = a.interleaved ? bid / 8 % a.q_c : bid % a.q_c;
+  const int pair0 = (a.interleaved ? bid / (8 * a.q_c) * 8 + bid % 8 : bid / a.q_c) * NP;
+  if (2 * pair0 >= a.n_groups) return;
 
   const uint16_t* planes = reinterpret_cast<const uint16_t*>(a.packed + kX3HeadFloats * 4) +
                            static_cast<int64_t>(q) * (RD / 32) * 9 * KS * kFragElems;
@@ -538,7 +545,8 @@ int x3_split(int64_t units) {
 
 template <int D, int RD>
 int launch_x3(const X3Args& a, int32_t n_pairs, int split, hipStream_t stream) {
-  const unsigned grid = static_cast<unsigned>(static_cast<int64_t>((n_pairs + 4 / split - 1) / (4 / split)) * a.q_c);
+  const int64_t blocks = (n_pairs + 4 / split - 1) / (4 / split);
+  const unsigned grid = static_cast<unsigned>((a.interleaved ? (blocks + 7) / 8 * 8 : blocks) * a.q_c);
   if (split == 4)
     hipLaunchKernelGGL((bigemm_fwd_x3_kernel<D, RD, 4>), dim3(grid), dim3(kX3Threads), 0, stream, a);
   else if (split == 2)
@@ -577,13 +585,13 @@ bool x3_forms_scales(int32_t batch, int32_t q_s, int32_t q_c) {
   return x3_split((static_cast<int64_t>(batch) * q_s + 1) / 2 * q_c) == 4;
 }
 
-int launch_fwd_x3(const float* x, float* out, const float* row_scale, bool norm, float eps, const void* packed,
+int launch_fwd_x3(const float* x, float* out, const float* row_scale, bool norm, float eps, bool interleaved, const void* packed,
                   const int32_t* tok, const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s,
                   int32_t q_c, int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream) {
   const int64_t groups = static_cast<int64_t>(batch) * q_s;
   if (groups >= (int64_t(1) << 31)) return fail(OW_ERR_UNSUPPORTED, "batch * token groups must be below 2^31");
   X3Args a{x, out, row_scale, static_cast<const uint8_t*>(packed), tok, chan, drop_scale, batch, n_tok, channels,
-           q_s, q_c, residual, static_cast<int32_t>(groups), norm ? 1 : 0, eps};
+           q_s, q_c, residual, static_cast<int32_t>(groups), norm ? 1 : 0, eps, interleaved ? 1 : 0};
   const int32_t n_pairs = static_cast<int32_t>((groups + 1) / 2);
   // A workgroup's offsets start at its first image: the images its 8 token groups can span.
   if (!x3_fits(n_tok, channels, q_s)) return fail(OW_ERR_UNSUPPORTED, "images too large for 32-bit offsets");

@@ -890,7 +890,7 @@ int pack_weights_x3(const void* a_u, const void* a_v, const void* a_o, const voi
                     const int32_t* channel_index, int32_t channels, int32_t q_c, int32_t d, int32_t rd, void* packed,
                     hipStream_t stream);
 bool x3_forms_scales(int32_t batch, int32_t q_s, int32_t q_c);  // no statistics pass: launch_fwd_x3 with norm
-int launch_fwd_x3(const float* x, float* out, const float* row_scale, bool norm, float eps, const void* packed, const int32_t* tok,
+int launch_fwd_x3(const float* x, float* out, const float* row_scale, bool norm, float eps, bool interleaved, const void* packed, const int32_t* tok,
                   const int32_t* chan, int32_t batch, int32_t n_tok, int32_t channels, int32_t q_s, int32_t q_c,
                   int32_t d, int32_t rd, int32_t residual, const float* drop_scale, hipStream_t stream);
 
