@@ -13,7 +13,7 @@
 // the operands of the first three products take 288 registers and the sums of the second three
 // 192.  Each value that crosses is written once and read twice (chan2_x3, reduce_x3).
 //
-// 28x28x256, B = 32 (100,352 slots of 64 channels): 81 + 78 + 52 us, where fp32 products of the
+// 28x28x256, B = 32 (100,352 slots of 64 channels): 81 + 73 + 51 us, where fp32 products of the
 // library around a gate kernel, gather, token mixings, per-tile outer products and the scatter took
 // 485; the whole step 640 -> 310 us.  With routed tiles X', dY written by a gather kernel first (27
 // us) the three took 80 + 72 + 51.  Errors against 64 bits over 4x4 to 56x56 images: dx 1.7e-7

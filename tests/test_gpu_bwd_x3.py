@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import omniwave_amd
+import omniwave_amd.block
 from omniwave_amd import _native
 from omniwave_amd.backward import bigemm_backward
 
@@ -83,3 +84,40 @@ def test_fp32_backward_against_float64(b, h, w, c, d, rd, route, level, drop) ->
         # a chain of at most 256 + 256 fp32 additions per product and six products deep, at random
         # signs: sqrt(512) half-ulps is 1.3e-6; cancellation in the gate's derivative within that
         assert rel(a, e) <= 2.0 ** -24 * 512 ** 0.5, name
+
+
+def _block(h, c, d, route, level):
+    torch.manual_seed(3)
+    block = omniwave_amd.block.OmniWeaveBlock(h, h, c, d, route, level).to(DEV)
+    with torch.no_grad():
+        block.gamma.fill_(1.0)
+    return block
+
+
+def test_empty_batch_has_zero_gradients() -> None:
+    block = _block(4, 64, 64, "local", 0)
+    x = torch.empty(0, 4, 4, 64, device=DEV, requires_grad=True)
+    grads = torch.autograd.grad(block(x), (x, *block.parameters()), torch.empty_like(x))
+    assert grads[0].shape == x.shape and all(not g.any() for g in grads[1:])
+
+
+def test_captured_step_replays_like_the_eager_one() -> None:
+    block = _block(7, 256, 128, "radix", 1)
+    x = torch.randn(9, 7, 7, 256, device=DEV).requires_grad_(True)
+    dy = torch.randn_like(x)
+    step = lambda: torch.autograd.grad(block(x), (x, *block.parameters()), dy)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = step()
+    for seed in range(3):
+        with torch.no_grad():
+            x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(seed)))
+        want = [g.clone() for g in step()]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(held, want))
