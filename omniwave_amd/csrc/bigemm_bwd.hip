@@ -33,7 +33,7 @@ namespace {
 constexpr float kLn2 = 0.6931471805599453f;
 
 // s = 1 / (1 + 2^U') with the hardware exp2 and reciprocal (each within about 1 ulp), as in the
-// forward's gate (silu_gate); the fp32 kernels divide exactly.
+// forward's gate (silu_gate) and the three-part fp32 kernels; the plain fp32 ones divide exactly.
 __device__ __forceinline__ float gate_sigmoid(float up) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(up));
 }
