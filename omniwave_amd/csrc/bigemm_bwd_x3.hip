@@ -259,12 +259,12 @@ chan_x3_kernel(ChanX3Args a) {
   };
   const uint32_t own = static_cast<uint32_t>(l32 * D + 4 * hh) * 4u;
   auto token_side = [&](const float(&raw)[MB][16], const X3& m, const __amdgpu_buffer_rsrc_t& out, X3(&op)[KS]) {
-    const X3 m0 = x3_keep_if(g0, m), m1 = x3_keep_if(!g0, m);
 #pragma unroll
     for (int cb = 0; cb < MB; ++cb) {
-      f32x16 p = x3_mma(x3_split8([&](int j) { return raw[cb][j]; }), m0, zero);
-      p = x3_mma(x3_split8([&](int j) { return raw[cb][8 + j]; }), m1, p);
+      const f32x16 p0 = x3_mma(x3_split8([&](int j) { return raw[cb][j]; }), m, zero);
+      const f32x16 p1 = x3_mma(x3_split8([&](int j) { return raw[cb][8 + j]; }), m, zero);
       mfma_drain();
+      const f32x16 p = pair_columns(g0, p0, p1);
 #pragma unroll
       for (int k = 0; k < 4; ++k) store4(out, own + static_cast<uint32_t>(32 * cb + 8 * k) * 4u, p, k);
       op[2 * cb] = x3_kstep(p, 0);
@@ -439,13 +439,12 @@ chan2_x3_kernel(ChanX3Args a) {
     }
 
   const X3 au = token_operand(a.a_u, true, l32, hh), av = token_operand(a.a_v, true, l32, hh);
-  const bool g0 = (lane & 16) == 0;
   int32_t row[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) row[i] = tab.row[wave][pair_token_row(i, hh)];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    f32x16 dx = zero;
+    f32x16 d0 = zero, d1 = zero;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
@@ -458,10 +457,11 @@ chan2_x3_kernel(ChanX3Args a) {
       for (int i = 0; i < 16; ++i) v[i] = scratch[pair_token_row(i, hh) * LD + l32];
       wave_lds_sync();
       const X3& t = m == 0 ? au : av;
-      dx = x3_mma(x3_keep_if(g0, t), x3_split8([&](int j) { return v[j]; }), dx);
-      dx = x3_mma(x3_keep_if(!g0, t), x3_split8([&](int j) { return v[8 + j]; }), dx);
+      d0 = x3_mma(t, x3_split8([&](int j) { return v[j]; }), d0);
+      d1 = x3_mma(t, x3_split8([&](int j) { return v[8 + j]; }), d1);
     }
     mfma_drain();
+    const f32x16 dx = pair_rows_of(d0, d1);
     const int32_t ch = a.chan[q * D + 32 * mb + l32];
     if (ch >= 0 && ch < a.channels) {
 #pragma unroll

@@ -3,8 +3,8 @@
 // (omniweave/models/block.py:83-108) for fp32 activations, any supported shape and route.
 //
 // A unit is one 32-token pair (two token groups) of one channel group, computed by the operand
-// scheme of ow_device.h (32x32x16 products, block-diagonal token matrices, accumulators reused
-// as the next operand) with every operand in three bf16 parts.  Every shape takes this one
+// scheme of ow_device.h (32x32x16 products, accumulators reused as the next operand) with every
+// operand in three bf16 parts and the groups' token products apart.  Every shape takes this one
 // kernel: x is read and out written by the lane that owns the channel, so contiguous, strided and
 // ragged groups differ only in the channel table.
 //
@@ -280,15 +280,15 @@ bigemm_fwd_x3_kernel(X3Args a) {
     }
 #pragma unroll
     for (int cb = 0; cb < MB; ++cb) {
-      f32x16 pu = zero, pv = zero;
+      f32x16 pg[2][2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
         const X3 xt = x3_split8([&](int j) { return raw[cb][8 * g + j] * sc[8 * g + j]; });
-        const bool mine = g == 0 ? g0 : !g0;
-        pu = x3_mma(xt, x3_keep_if(mine, au), pu);
-        pv = x3_mma(xt, x3_keep_if(mine, av), pv);
+        pg[0][g] = x3_mma(xt, au, zero);
+        pg[1][g] = x3_mma(xt, av, zero);
       }
       mfma_drain();
+      const f32x16 pu = pair_columns(g0, pg[0][0], pg[0][1]), pv = pair_columns(g0, pg[1][0], pg[1][1]);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         Pu[2 * cb + s] = x3_kstep(pu, s);
@@ -477,16 +477,16 @@ bigemm_fwd_x3_kernel(X3Args a) {
   mfma_drain();
 
   // delta = A_o W, residual and routed store of one 32-channel block.
-  const X3 ao = token_operand(2), ao0 = x3_keep_if(g0, ao), ao1 = x3_keep_if(!g0, ao);
+  const X3 ao = token_operand(2);
   float ds[2] = {1.0f, 1.0f};
   if (a.drop_scale) {
 #pragma unroll
     for (int g = 0; g < 2; ++g) ds[g] = a.drop_scale[min(2 * (pair0 + pl) + g, a.n_groups - 1) / a.q_s];
   }
   auto store = [&](uint32_t ch, const f32x16& w, float(&xv)[16]) {
-    f32x16 dl = x3_mma(ao0, x3_kstep(w, 0), zero);
-    dl = x3_mma(ao1, x3_kstep(w, 1), dl);
+    const f32x16 d0 = x3_mma(ao, x3_kstep(w, 0), zero), d1 = x3_mma(ao, x3_kstep(w, 1), zero);
     mfma_drain();
+    f32x16 dl = pair_rows_of(d0, d1);
     if (a.drop_scale) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) dl[i] *= ds[i >> 3];

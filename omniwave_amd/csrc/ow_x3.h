@@ -48,10 +48,6 @@ __device__ __forceinline__ X3 x3_kstep(const f32x16& acc, int s) {
   return x3_split8([&](int j) { return acc[8 * s + j]; });
 }
 
-__device__ __forceinline__ X3 x3_keep_if(bool keep, const X3& v) {
-  return X3{{keep_if(keep, v.p[0]), keep_if(keep, v.p[1]), keep_if(keep, v.p[2])}};
-}
-
 // c + a b, smallest products first.
 __device__ __forceinline__ f32x16 x3_mma(const X3& a, const X3& b, f32x16 c) {
   c = BF16::mma32(a.p[2], b.p[0], c);
@@ -71,6 +67,25 @@ __device__ __forceinline__ void x3_mma_apart(const X3& a, const X3& b, f32x16& h
   lo = BF16::mma32(a.p[1], b.p[0], lo);
   lo = BF16::mma32(a.p[0], b.p[1], lo);
   hi = BF16::mma32(a.p[0], b.p[0], hi);
+}
+
+// The two token groups of a pair share a product's 32 rows and columns but not its K steps: each
+// group's product is formed apart, with the same token matrix in every lane, and its half of the
+// result taken.  (A zero in the other group's place would be as many products, but 0 x NaN and
+// 0 x Inf are NaN, and the groups of a pair can belong to different images.)
+// lane & 15 = token (columns): group 0 in lanes without bit 4.
+__device__ __forceinline__ f32x16 pair_columns(bool group0, const f32x16& p0, const f32x16& p1) {
+  f32x16 r;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = group0 ? p0[i] : p1[i];
+  return r;
+}
+// rows = tokens: group 0 in registers 0 to 7 (pair_token_row).
+__device__ __forceinline__ f32x16 pair_rows_of(const f32x16& p0, const f32x16& p1) {
+  f32x16 r;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = i < 8 ? p0[i] : p1[i];
+  return r;
 }
 
 }  // namespace ow
