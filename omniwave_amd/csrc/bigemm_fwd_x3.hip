@@ -105,6 +105,12 @@ __global__ void __launch_bounds__(256) pack_x3_kernel(PackX3Args p) {
   for (int n = 0; n < 3; ++n) dst[64 * n] = uint4{w[n][0], w[n][1], w[n][2], w[n][3]};
 }
 
+// The gate with silu(U) formed before V comes in: a large U V beside a vanishing sigmoid is zero,
+// where (U V) s (silu_gate) overflows.
+__device__ __forceinline__ float silu_first(float up, float vp) {
+  return up * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(up)) * vp;
+}
+
 struct X3Args {
   const float* x;
   float* out;
@@ -395,7 +401,7 @@ bigemm_fwd_x3_kernel(X3Args a) {
   auto gate_all = [&] {
     f32x16 z;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = silu_gate(U[i], V[i]);
+    for (int i = 0; i < 16; ++i) z[i] = silu_first(U[i], V[i]);
     Z[0] = x3_kstep(z, 0);
     Z[1] = x3_kstep(z, 1);
   };
@@ -435,13 +441,10 @@ bigemm_fwd_x3_kernel(X3Args a) {
         if constexpr (decltype(j)::value == 0) {
           for (int h = 0; h < 2; ++h) den[h] = u0[2 * k + h];
           pin(den);
-          for (int h = 0; h < 2; ++h) {
-            num[h] = den[h] * v0[2 * k + h];
-            den[h] = 1.0f + __builtin_amdgcn_exp2f(den[h]);
-          }
+          for (int h = 0; h < 2; ++h) den[h] = 1.0f + __builtin_amdgcn_exp2f(den[h]);
         } else if constexpr (decltype(j)::value == 1) {
           pin(den);
-          for (int h = 0; h < 2; ++h) num[h] *= __builtin_amdgcn_rcpf(den[h]);
+          for (int h = 0; h < 2; ++h) num[h] = u0[2 * k + h] * __builtin_amdgcn_rcpf(den[h]) * v0[2 * k + h];  // as silu_first
         } else {
           pin(num);
           uint32_t p0, p1, p2;

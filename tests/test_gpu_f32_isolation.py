@@ -106,3 +106,15 @@ def test_backward_keeps_groups_apart(b, h, w, c, d, rd, route, level, value, whe
         dx = lambda g, t: bigemm_backward(g, t, weight, *args, flags, EPS)[0].view(b, h * w, c)
         want, got = dx(dy, x), dx(bad["dy"], bad["x"])
         assert torch.equal(got[keep], want[keep])
+
+
+def test_gate_of_large_products() -> None:
+    """U far below zero beside a V so large that U V overflows: silu(U) is zero and so is delta.
+    A = I, every weight of B_u -1e20 / d and of B_v 1e20 / d: U = -1e20, V = 1e20 for x = 1."""
+    d, c, rd = 128, 128, 256
+    plan = omniwave_amd.build_route_plan(8, 8, c, G, d, "local", 0)
+    eye = torch.eye(G, device=DEV)
+    b_u = torch.full((1, d, rd), -1e20 / d, device=DEV)
+    delta = bigemm_delta_hip(x=torch.ones(2, 8, 8, c, device=DEV), plan=plan, a_u=eye, a_v=eye, a_o=eye, b_u=b_u, b_v=-b_u,
+                             b_o=torch.ones(1, rd, d, device=DEV), gamma=torch.ones(c, device=DEV))
+    assert not delta.any()
