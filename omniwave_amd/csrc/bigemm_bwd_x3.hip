@@ -83,11 +83,7 @@ __global__ void __launch_bounds__(kThreads) pack_bwd_x3_kernel(PackBwdX3Args p) 
       v *= weight64(p.b[kind], mat + (kind < 2 ? static_cast<int64_t>(c) * p.rd + e : static_cast<int64_t>(e) * p.d + c),
                     p.wdtype);
 #pragma unroll
-      for (int n = 0; n < 3; ++n) {
-        const uint16_t b = BF16::from_f32(static_cast<float>(v));
-        part[n][h] = b;
-        v -= static_cast<double>(BF16::to_f32(b));
-      }
+      for (int n = 0; n < 3; ++n) part[n][h] = x3_part(v, n);
     }
 #pragma unroll
     for (int n = 0; n < 3; ++n) w[n][j2] = part[n][0] | (part[n][1] << 16);
@@ -122,7 +118,7 @@ struct ChanX3Args {
 // Row l32 % 16 of a token matrix (or of its transpose), 8 entries in the K order of the pair scheme.
 __device__ __forceinline__ X3 token_operand(const float* m, bool transposed, int l32, int hh) {
   const int r = l32 & 15;
-  return x3_split8([&](int j) {
+  return x3_split8<true>([&](int j) {
     const int k = pair_token_row(j, hh);
     return transposed ? m[k * kG + r] : m[r * kG + k];
   });
@@ -261,8 +257,8 @@ chan_x3_kernel(ChanX3Args a) {
   auto token_side = [&](const float(&raw)[MB][16], const X3& m, const __amdgpu_buffer_rsrc_t& out, X3(&op)[KS]) {
 #pragma unroll
     for (int cb = 0; cb < MB; ++cb) {
-      const f32x16 p0 = x3_mma(x3_split8([&](int j) { return raw[cb][j]; }), m, zero);
-      const f32x16 p1 = x3_mma(x3_split8([&](int j) { return raw[cb][8 + j]; }), m, zero);
+      const f32x16 p0 = x3_mma(x3_split8<true>([&](int j) { return raw[cb][j]; }), m, zero);
+      const f32x16 p1 = x3_mma(x3_split8<true>([&](int j) { return raw[cb][8 + j]; }), m, zero);
       mfma_drain();
       const f32x16 p = pair_columns(g0, p0, p1);
 #pragma unroll
@@ -405,7 +401,7 @@ chan2_x3_kernel(ChanX3Args a) {
       for (int s = 0; s < 2; ++s) {
         const float* p = scratch + l32 * LD + 16 * s + 4 * hh;
         const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 8);
-        use(2 * mb + s, x3_split8([&](int j) { return j < 4 ? lo[j & 3] : hi[j & 3]; }));
+        use(2 * mb + s, x3_split8<true>([&](int j) { return j < 4 ? lo[j & 3] : hi[j & 3]; }));
       }
       wave_lds_sync();
     }

@@ -91,11 +91,7 @@ __global__ void __launch_bounds__(256) pack_x3_kernel(PackX3Args p) {
                           (kind < 2 ? static_cast<int64_t>(c) * p.rd + e : static_cast<int64_t>(e) * p.d + c);
       v *= static_cast<double>(load_weight(kind == 0 ? p.b_u : kind == 1 ? p.b_v : p.b_o, src, p.wdtype));
 #pragma unroll
-      for (int n = 0; n < 3; ++n) {
-        const uint16_t b = BF16::from_f32(static_cast<float>(v));
-        part[n][h] = b;
-        v -= static_cast<double>(BF16::to_f32(b));
-      }
+      for (int n = 0; n < 3; ++n) part[n][h] = x3_part(v, n);
     }
 #pragma unroll
     for (int n = 0; n < 3; ++n) w[n][j2] = part[n][0] | (part[n][1] << 16);
@@ -228,7 +224,7 @@ bigemm_fwd_x3_kernel(X3Args a) {
     const float* p = head + m * kG * kG;
     const float4 lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 8);
     const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    return x3_split8([&](int j) { return v[j]; });
+    return x3_split8<true>([&](int j) { return v[j]; });
   };
   const bool g0 = (lane & 16) == 0;
   __syncthreads();
@@ -289,7 +285,7 @@ bigemm_fwd_x3_kernel(X3Args a) {
       f32x16 pg[2][2];
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        const X3 xt = x3_split8([&](int j) { return raw[cb][8 * g + j] * sc[8 * g + j]; });
+        const X3 xt = x3_split8<true>([&](int j) { return raw[cb][8 * g + j] * sc[8 * g + j]; });
         pg[0][g] = x3_mma(xt, au, zero);
         pg[1][g] = x3_mma(xt, av, zero);
       }

@@ -21,26 +21,42 @@ __device__ __forceinline__ X3 x3_zero() {
   return X3{{z, z, z}};
 }
 
-// Two fp32 values -> their three parts, packed (first value in the low half).
+// Two fp32 values -> their three parts, packed (first value in the low half).  The largest values
+// (from 3.3962e38 on) round up to infinity in bf16; kWhole keeps them: the first part is at most
+// bf16's largest and the second holds the rest.  It is for the caller's tensors (weights: x3_part); for the
+// sums in between, where those values are infinite, it would cost 2% of the whole kernels.
+constexpr float kMostBf16 = 3.38953139e38f;  // 0x7f7f0000
+template <bool kWhole = false>
 __device__ __forceinline__ void x3_split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
-  p0 = BF16::pack2(a, b);
+  if constexpr (kWhole)
+    p0 = BF16::pack2(__builtin_amdgcn_fmed3f(a, -kMostBf16, kMostBf16), __builtin_amdgcn_fmed3f(b, -kMostBf16, kMostBf16));
+  else
+    p0 = BF16::pack2(a, b);
   const float a1 = a - __uint_as_float(p0 << 16), b1 = b - __uint_as_float(p0 & 0xffff0000u);
   p1 = BF16::pack2(a1, b1);
   p2 = BF16::pack2(a1 - __uint_as_float(p1 << 16), b1 - __uint_as_float(p1 & 0xffff0000u));
 }
 
-template <class V>
+template <bool kWhole = false, class V>
 __device__ __forceinline__ X3 x3_split8(V v) {  // v(j), j = 0..7
   X3 r;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     uint32_t a, b, c;
-    x3_split2(v(2 * q), v(2 * q + 1), a, b, c);
+    x3_split2<kWhole>(v(2 * q), v(2 * q + 1), a, b, c);
     r.p[0][q] = a;
     r.p[1][q] = b;
     r.p[2][q] = c;
   }
   return r;
+}
+
+// Part n of a folded weight, taken off it (only the first is cut off, so that NaN stays NaN).
+__device__ __forceinline__ uint16_t x3_part(double& v, int n) {
+  const float f = static_cast<float>(v);
+  const uint16_t b = BF16::from_f32(n == 0 ? __builtin_amdgcn_fmed3f(f, -kMostBf16, kMostBf16) : f);
+  v -= static_cast<double>(BF16::to_f32(b));
+  return b;
 }
 
 // Accumulator registers 8s..8s+7 as an operand (K step s of the next product).

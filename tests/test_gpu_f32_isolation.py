@@ -108,6 +108,56 @@ def test_backward_keeps_groups_apart(b, h, w, c, d, rd, route, level, value, whe
         assert torch.equal(got[keep], want[keep])
 
 
+# Tensor of the largest values, and the scales of others that keep every product and sum a number.
+LARGE = [("x", {"a_u": -30, "a_v": -30, "b_u": -98, "b_v": -98}), ("b_o", {"b_u": -35, "b_v": -35}),
+         ("a_o", {"b_o": -60})]
+
+
+def _large(t):
+    """Values of either sign that round up to infinity in bf16."""
+    gen = torch.Generator().manual_seed(6)
+    sign = torch.where(torch.rand(t.shape, generator=gen) < 0.5, -1.0, 1.0)
+    big = sign * LARGEST * (1.0 - 2.0 ** -10 * torch.rand(t.shape, generator=gen))
+    assert big.bfloat16().isinf().all()
+    return big.to(DEV)
+
+
+@pytest.mark.parametrize("name,scales", LARGE, ids=[name for name, _ in LARGE])
+@pytest.mark.parametrize("d,c", [(128, 512), (64, 256)])
+def test_largest_values_are_numbers(d, c, name, scales) -> None:
+    """delta with one tensor of the largest fp32 values against float64."""
+    plan, p, _, x, _ = _inputs(2, 14, 14, c, d, 2 * d, "local", 0)
+    w = {k: v * 2.0 ** scales.get(k, 0) for k, v in {**p, "x": x, "gamma": torch.ones(c, device=DEV)}.items()}
+    w[name] = _large(w[name])
+    x = w.pop("x")
+    got = bigemm_delta_hip(x=x, plan=plan, **w).cpu().double()
+    tok = torch.as_tensor(plan.token_indices).long().reshape(-1)
+    n = 14 * 14
+    live = (tok >= 0) & (tok < n)
+    t = x.double().cpu().view(2, n, c)[:, tok.clamp(0, n - 1)] * live[:, None]
+    t = t.reshape(2, -1, G, c // d, d).permute(0, 1, 3, 2, 4)
+    w64 = {k: v.double().cpu() for k, v in w.items()}
+    u, v = w64["a_u"] @ t @ w64["b_u"], w64["a_v"] @ t @ w64["b_v"]
+    o = w64["a_o"] @ (torch.nn.functional.silu(u) * v @ w64["b_o"])
+    o = o.permute(0, 1, 3, 2, 4).reshape(2, -1, c)
+    want = torch.zeros(2, n, c, dtype=torch.float64).index_copy(1, tok[live], o[:, live])
+    assert got.isfinite().all()
+    # the bound of the three-part forward (sqrt(4 * 96) roundings of 2^-24)
+    assert (got.view(2, n, c) - want).norm() <= 1.2e-6 * want.norm()
+
+
+@pytest.mark.parametrize("name,scales", [LARGE[0], ("dy", {"a_o": -100, "b_o": -60})], ids=["x", "dy"])
+@pytest.mark.parametrize("d,c", [(128, 512), (64, 256)])
+def test_largest_values_have_gradients(d, c, name, scales) -> None:
+    """Gradients of the operator that are numbers."""
+    plan, p, _, x, dy = _inputs(2, 14, 14, c, d, 2 * d, "local", 0)
+    w = {k: v * 2.0 ** scales.get(k, 0) for k, v in {**p, "x": x, "dy": dy}.items()}
+    w[name] = _large(w[name])
+    grads = bigemm_backward(w["dy"], w["x"], None, w["gamma"], w["a_u"], w["a_v"], w["a_o"], w["b_u"], w["b_v"], w["b_o"],
+                            plan, 0, EPS)
+    assert grads[1] is None and all(g.isfinite().all() for g in grads[:1] + grads[2:])
+
+
 def test_gate_of_large_products() -> None:
     """U far below zero beside a V so large that U V overflows: silu(U) is zero and so is delta.
     A = I, every weight of B_u -1e20 / d and of B_v 1e20 / d: U = -1e20, V = 1e20 for x = 1."""
