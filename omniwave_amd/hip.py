@@ -331,7 +331,7 @@ def _forward(x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o, plan, flags: i
     if not _plain(*tensors, drop_scale):
         return bigemm_fwd(*tensors, _plan_desc(plan), flags, eps, drop_scale, want_scales)[0]
     geo = _geometry(plan_key(plan))
-    if torch.is_grad_enabled() and any([t is not None and t.requires_grad for t in tensors]):
+    if torch.is_grad_enabled() and any([t is not None and t.requires_grad for t in (*tensors, drop_scale)]):
         return _PlainForward.apply(*tensors, geo, flags, eps, drop_scale, want_scales)
     return _run_forward(*tensors, geo, flags, eps, drop_scale, want_scales)[0]
 
@@ -626,7 +626,9 @@ def _chain(x, stats_in, norm_weight, plan, a_u, a_v, a_o, b_u, b_v, b_o, gamma, 
         raise RuntimeError("bigemm_block_chain_hip is inference-only (no backward); run it under torch.no_grad()")
     flags = _native.OW_FUSE_NORM | _native.OW_FUSE_RESIDUAL | (_native.OW_FUSE_FP8 if fp8 else 0)
     tensors = (x, norm_weight, gamma, a_u, a_v, a_o, b_u, b_v, b_o)
-    if _plain(*tensors, stats_in):
+    # Gradients of the other inputs: the operator, whose backward raises.
+    tracked = torch.is_grad_enabled() and any([t is not None and t.requires_grad for t in (a_v, a_o, b_v, b_o, stats_in)])
+    if not tracked and _plain(*tensors, stats_in):
         out, stats, wrote = _run_chain(*tensors, _geometry(plan_key(plan)), flags, float(eps), stats_in, int(factor), True)
     else:
         out, stats, written = bigemm_fwd_chain(*tensors, _plan_desc(plan), flags, float(eps), stats_in, int(factor))
