@@ -525,7 +525,7 @@ int ow_small_to_f32(const void* const* src, const int32_t* dtype, const int64_t*
  * omniweave/ops/triton.py:256-292), for d = 128 and for d = 64 with batch * Q_s even:
  * ow_bwd_block_workspace returns the bytes it needs (drop, scales: whether drop_scale and
  * row_scale will be given), or 0 when the shape or dtype has no such path and the caller composes
- * the entry points above (fp32, d = 64 with an odd number of token groups).
+ * the entry points above (fp32, d = 64 with an odd number of token groups, an empty batch).
  *   grad, x      [B, H*W, C] of dtype; small: norm weight (NULL without OW_FUSE_NORM), gamma,
  *                A_u, A_v, A_o with their dtypes; b_u, b_v, b_o of weight_dtype, contiguous
  *   row_scale    the forward's RMSNorm scales (ow_bigemm_fwd_scales), or NULL: formed here

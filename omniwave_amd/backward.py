@@ -227,17 +227,20 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
     of ``_cast_grads``) and, with ``want_cast`` and parameters of one 16-bit dtype, that buffer in
     their dtype (else None).  bf16 / fp16 shapes with kernels of their own run as one native call
     (``ow_bwd_block``); the rest is composed here."""
-    lib = _native.lib()
     dev = x.device
     dtype = x.dtype
-    code = _DTYPE_CODE[dtype]
     fuse_norm = bool(flags & _native.OW_FUSE_NORM)
     residual = bool(flags & _native.OW_FUSE_RESIDUAL)
     x = x.contiguous()
-    if grad.dtype != dtype or not grad.is_contiguous():
-        grad = grad.to(dtype).contiguous()
     batch = x.shape[0]
     q_c, d, rd = b_u.shape
+    n_grads = 768 + 3 * q_c * d * rd + (2 if fuse_norm else 1) * plan.channels
+    if batch == 0:  # no kernel takes one: nothing is summed
+        return torch.empty_like(x), torch.zeros(n_grads, dtype=torch.float32, device=dev), None
+    lib = _native.lib()
+    code = _DTYPE_CODE[dtype]
+    if grad.dtype != dtype or not grad.is_contiguous():
+        grad = grad.to(dtype).contiguous()
     q_s = plan.token_indices.shape[0]
     slots = batch * q_s * 16
     n_rows = batch * plan.height * plan.width
@@ -256,11 +259,10 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
     if nbytes:
         small = [(t if t.is_contiguous() else t.contiguous()) if t.device == dev and t.dtype in _DTYPE_CODE
                  else _fp32(t, dev) for t in (norm_weight if fuse_norm else gamma, gamma, a_u, a_v, a_o)]
-        n = 768 + 3 * q_c * d * rd + (2 if fuse_norm else 1) * plan.channels
-        g_all = torch.empty(n, dtype=torch.float32, device=dev)
+        g_all = torch.empty(n_grads, dtype=torch.float32, device=dev)
         dts = {t.dtype for t in ((norm_weight,) if fuse_norm else ()) + (gamma, a_u, a_v, a_o, b_u, b_v, b_o)}
         cast_dtype = dts.pop() if len(dts) == 1 else None
-        cast = (torch.empty(n, dtype=cast_dtype, device=dev)
+        cast = (torch.empty(n_grads, dtype=cast_dtype, device=dev)
                 if want_cast and cast_dtype in (torch.bfloat16, torch.float16) else None)
         scale = drop_scale.to(device=dev, dtype=torch.float32).contiguous() if drop_scale is not None else None
         rscale = row_scale.to(device=dev, dtype=torch.float32).contiguous() if row_scale is not None else None
@@ -298,9 +300,7 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
     # The fp32 parameter gradients in one buffer (the token matrices, B_u, B_v, B_o, then gamma
     # and the norm weight: every block that a kernel sums into starts 16-byte aligned), so that
     # parameters of one dtype are cast back with one kernel.
-    n_c = (2 if fuse_norm else 1) * plan.channels
-    nb = q_c * d * rd
-    g_all = torch.empty(768 + 3 * nb + n_c, dtype=torch.float32, device=dev)
+    g_all = torch.empty(n_grads, dtype=torch.float32, device=dev)
     g_a = g_all[:768].view(3, 256)
 
     with torch.cuda.device(dev):
@@ -377,6 +377,7 @@ def _backward_once(grad: Tensor, x: Tensor, norm_weight: Tensor | None, gamma: T
 
         # Parameter gradients from the folded ones, into g_all (every element is written: each
         # channel of the permutation exactly once).
+        nb = q_c * d * rd
         g_b = g_all[768:768 + 3 * nb]
         g_bu, g_bv = g_b[:nb].view(q_c, d, rd), g_b[nb:2 * nb].view(q_c, d, rd)
         g_bo = g_b[2 * nb:].view(q_c, rd, d)
@@ -406,9 +407,6 @@ def _backward_x3(lib, grad: Tensor, grad_delta: Tensor, x: Tensor, rscale: Tenso
     n_tok, channels = plan.height * plan.width, plan.channels
     n_rows = batch * n_tok
     dx = torch.empty_like(x)
-    if n_rows == 0:
-        g_all.zero_()
-        return dx
     f32 = _DTYPE_CODE[torch.float32]
     nd, nr, nb = q_c * slots * d, q_c * slots * rd, q_c * d * rd
     packed_bytes = lib.ow_bwd_x3_packed_bytes(q_c, d, rd)

@@ -36,11 +36,11 @@ struct BwdPlan {
   size_t delta, rscale, small, xt, dyt, wpk, pu, pv, dw, z, du, dv, partial, red, gb, g, dxt, total;
 };
 
-// Whether the shape has kernels of its own (d = 64 in pairs of token groups, d = 128), and the
-// workspace layout.
+// Whether the shape has kernels of its own (d = 64 in pairs of token groups, d = 128; no empty
+// batch, whose sums have no rows), and the workspace layout.
 bool bwd_plan(const OwPlan* plan, int32_t batch, int32_t rd, int32_t dtype, int32_t flags, bool drop, bool scales,
               BwdPlan& p) {
-  if (!plan || batch < 0 || (dtype != OW_DTYPE_BF16 && dtype != OW_DTYPE_F16) || plan->spatial_tile != kG) return false;
+  if (!plan || batch < 1 || (dtype != OW_DTYPE_BF16 && dtype != OW_DTYPE_F16) || plan->spatial_tile != kG) return false;
   if (ow_plan_dims(plan, &p.q_s, &p.q_c) != OW_OK) return false;
   p.d = plan->channel_tile;
   p.rd = rd;
