@@ -295,10 +295,12 @@ _PLAIN = (Tensor, torch.nn.Parameter)
 def _plain(*tensors: Tensor | None) -> bool:
     """Whether a call may skip the torch.library dispatcher, which costs more than a small launch:
     plain tensors with nothing around the call that has to see the operator (compilation, tracing,
-    torch function or dispatch modes, functorch transforms such as vmap, forward-mode gradients)."""
+    torch function or dispatch modes, functorch transforms such as vmap, forward-mode gradients, a
+    profiler, whose records name the operator)."""
     if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0):
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._autograd._profiler_enabled()):
         return False
     for t in tensors:
         if t is not None and type(t) not in _PLAIN:

@@ -44,6 +44,15 @@ def test_nothing_that_must_see_the_operator_is_passed_by() -> None:
     assert _plain(t)
 
 
+def test_a_profiler_sees_the_operator() -> None:
+    t = torch.ones(3)
+    with torch.autograd.profiler.profile():
+        assert not _plain(t)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        assert not _plain(t)
+    assert _plain(t)
+
+
 PARAMS = ("norm_weight", "a_u", "a_v", "a_o", "b_u", "b_v", "b_o", "gamma")
 
 
