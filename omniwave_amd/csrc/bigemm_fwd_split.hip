@@ -14,7 +14,9 @@
 //     chunks in order: the 32x32 blocks of W are independent, so no partial sums are added;
 //   * block w of delta^T, staged through LDS, leaves as 16-byte pieces of the rows the wave
 //     loaded (2-byte elements for strided groups).
-// Bound by the latency of its loads and by the chain rows -> P -> Z -> W.
+// Bound by the latency of its loads and by the chain rows -> P -> Z -> W: at 7x7x1024 radix 1, B = 8
+// waves wait for memory or LDS 47% of their time and the matrix cores are busy 2%.  Every instance
+// uses all 256 registers of two waves per SIMD and spills four more (20 bytes of scratch a lane).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -288,14 +290,13 @@ void launch_stride(const PersistArgs& a, dim3 g, hipStream_t stream) {
 
 }  // namespace
 
-// Up to 640 pairs x groups: two workgroups fit on a CU, and the second round of a larger launch
-// takes as long as the persistent kernel (block, us, split against persistent, the latter with
+// Up to two and a half pairs x groups per CU (640 on 256 CUs): two workgroups fit on a CU, and the
+// second round of a larger launch takes as long as the persistent kernel (block, us, split against persistent, the latter with
 // its statistics pass: 14x14x512 local B = 1: 7.0 / 17.0, B = 16 (416): 10.7 / 18.1, B = 20 (520):
 // 14.5 / 18.2, B = 32 (832): 18.9 / 18.9; 7x7x1024 radix 1 B = 8 (128): 9.4 / 25.6, B = 32 (512):
 // 17.8 / 25.8, B = 64 (1024): 31.2 / 27.2).
 bool split_supported(int64_t n_groups, int32_t q_c) {
-  constexpr int64_t kSplitMost = 640;
-  return (n_groups + 1) / 2 * q_c <= kSplitMost;
+  return 2 * ((n_groups + 1) / 2 * q_c) <= 5 * static_cast<int64_t>(device_cus());
 }
 
 int launch_fwd_split(const PersistArgs& a, int32_t dtype, hipStream_t stream) {
