@@ -81,15 +81,6 @@ def _tile_outer(lib, in1: Tensor, in2: Tensor, d: int, code: int, stream: int) -
     return partial.sum(dim=2)
 
 
-def _sum_rows(lib, partial: Tensor, rows: int, out: Tensor, stream: int) -> None:
-    """out = the sum of the ``rows`` equal-sized row blocks of the fp32 buffer ``partial``
-    (``ow_sum_rows``: a fixed summation order, so replays and reruns give identical bits).
-    Both buffers are contiguous fp32 and start 16-byte aligned."""
-    cols = out.numel()
-    assert partial.is_contiguous() and out.is_contiguous() and partial.numel() == rows * cols
-    _native.check(lib.ow_sum_rows(partial.data_ptr(), rows, cols, out.data_ptr(), stream), "ow_sum_rows")
-
-
 def _slot_reduce(a: Tensor, b: Tensor) -> Tensor:
     """sum over slots of a^T b per channel group ([q_c, S, m] x [q_c, S, n] -> fp32 [q_c, m, n]).
 
@@ -412,8 +403,8 @@ def _backward_x3(lib, grad: Tensor, grad_delta: Tensor, x: Tensor, rscale: Tenso
     packed_bytes = lib.ow_bwd_x3_packed_bytes(q_c, d, rd)
     n_part = lib.ow_bwd_channel_x3_partials(slots, q_c)
     ranges = lib.ow_bwd_param_reduce_x3_ranges(slots, q_c)
-    # One buffer: P_u, P_v, dW', Z, dU', dV', g, the partial sums, the folded-weight
-    # gradients and the packed weights (every size but g's and the last a multiple of 16 bytes).
+    # One buffer: P_u, P_v, dW', Z, dU', dV', the partial sums, the folded-weight gradients, the
+    # packed weights, and g last (its size alone need not be a multiple of 16 bytes).
     sizes = [nd] * 3 + [nr] * 3 + [768 * n_part, ranges * 3 * nb, 3 * nb, packed_bytes // 4, n_rows * channels]
     work = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
     ptr = [work.data_ptr()]

@@ -5,6 +5,11 @@
 //     a b = a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0)      (fp32 accumulation)
 // What is left out (a1 b2, a2 b1, a2 b2) is below 2^-25 of the product.  The bf16 MFMAs have 16
 // times the rate of the fp32 ones, so six of them cost 0.375 of one fp32 product.
+//
+// Range: up to fp32's largest value (x3_split2).  Parts end at bf16's smallest subnormal, so an
+// operand below about 2^-110 is held to 2^-134 instead of 24 bits (gradients from an upstream of
+// 2^-112: 5e-7 off, 2^-116: 7e-6).  An infinite operand makes its token group's results NaN (its
+// parts are not all infinite), never another group's.
 #pragma once
 
 #include "ow_device.h"
@@ -15,11 +20,6 @@ namespace ow {
 struct X3 {
   u32x4 p[3];
 };
-
-__device__ __forceinline__ X3 x3_zero() {
-  const u32x4 z = {0u, 0u, 0u, 0u};
-  return X3{{z, z, z}};
-}
 
 // Two fp32 values -> their three parts, packed (first value in the low half).  The largest values
 // (from 3.3962e38 on) round up to infinity in bf16; kWhole keeps them: the first part is at most

@@ -27,7 +27,7 @@ import torch
 from torch import Tensor
 
 from omniwave_amd import _native
-from omniwave_amd.routing import (RoutePlan, build_route_plan, device_tables, native_plan, plan_key, plan_tiles,
+from omniwave_amd.routing import (RoutePlan, build_route_plan, device_tables, native_plan, plan_key,
                                   s2d_rows_table)
 
 SPATIAL_TILE = 16
