@@ -300,7 +300,7 @@ def _plain(*tensors: Tensor | None) -> bool:
     if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._autograd._profiler_enabled()):
+            or torch.autograd.profiler._is_profiler_enabled):
         return False
     for t in tensors:
         if t is not None and type(t) not in _PLAIN:

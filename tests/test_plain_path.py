@@ -50,6 +50,13 @@ def test_a_profiler_sees_the_operator() -> None:
         assert not _plain(t)
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
         assert not _plain(t)
+    steps = torch.profiler.schedule(wait=1, warmup=0, active=1, repeat=1)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], schedule=steps) as prof:
+        plain = []
+        for _ in range(3):  # waiting, recording, done
+            plain.append(_plain(t))
+            prof.step()
+    assert plain == [True, False, True]
     assert _plain(t)
 
 
